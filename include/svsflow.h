@@ -286,9 +286,31 @@ int svs_tvl1_plan_set_shape(svs_plan* plan, int level, int bx, int by, int cz, v
  * graph: mode 1 runs each warp's iterations in one resident launch (one
  * work-group per instance holding the state on chip; only for levels whose
  * instances have at most 2048 voxels), 0 launches the marching sweep once per
- * iteration, -1 restores the automatic choice (resident wherever the level
- * qualifies).  Results do not depend on the mode.  No reference counterpart. */
+ * iteration, -1 restores the automatic choice (resident or block-resident
+ * wherever the level qualifies).  Results do not depend on the mode.  No reference counterpart. */
 int svs_tvl1_plan_set_resident(svs_plan* plan, int level, int mode, void* stream);
+
+/* How a level runs the block-resident sweep (all iterations of a warp in one
+ * launch, an instance's state held on chip by several work-groups that
+ * exchange their faces): out[0..4] = instances it runs (0: the level does not
+ * use it), voxels per thread, work-groups of its largest instance, launches
+ * per warp, and how often an instance of the plan had to be redone by one
+ * work-group (see svs_tvl1_plan_set_wait_limit; waits for the plan's enqueued
+ * work).  It is used wherever it applies: more than 2048 voxels per
+ * instance, an instance's tiles on chip at once (about 520,000 voxels), the
+ * reference's model, no statistics, no pinned sweep shape.  mode 0 of
+ * svs_tvl1_plan_set_resident and svs_tvl1_plan_set_shape switch it off for a
+ * level, mode -1 on again.  No reference counterpart. */
+int svs_tvl1_plan_blocks(const svs_plan* plan, int level, int* out);
+
+/* The longest a work-group of the block-resident sweep waits for a neighbour
+ * (default 0.2 s) before its instance's iterations are redone by one
+ * work-group alone, slowly and with the same results; the plan's later runs
+ * then use the marching sweep, until mode -1 of svs_tvl1_plan_set_resident.
+ * That happens only when something keeps the device from holding an
+ * instance's work-groups at the same time, such as another process's kernels.
+ * No reference counterpart. */
+int svs_tvl1_plan_set_wait_limit(svs_plan* plan, int microseconds, void* stream);
 
 /* Per-iteration statistics, the reference's residual norms made usable:
  * tvl13d.py:222, 237 and 253 compute ||p^{n+1} - p^n||, ||u^{n+1} - u^n|| and

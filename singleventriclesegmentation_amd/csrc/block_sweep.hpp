@@ -1,0 +1,738 @@
+// The block-resident sweep: all K primal-dual iterations of one warp in one
+// launch, for instances whose whole state fits the chip.  Included by
+// solver.hip (LevelDesc is its descriptor table).
+//
+// An instance is cut into tiles of at most V * 512 voxels, one work-group of
+// 512 threads per tile.  A thread owns up to V voxels and keeps their u, p,
+// (s, n) and (rho_c, g) in registers for the whole warp; LDS holds what
+// neighbours read, u and the derivative columns of r = D p', with a one-voxel
+// halo.  HBM is read once per warp and written once; per iteration only the
+// tile faces travel, 24 bytes per face voxel (3 components of u, then the 3 of
+// r across that face):
+//   1. dual step from u and its halo; own r -> LDS;            barrier
+//   2. send the faces of r, receive the neighbours';           barrier
+//   3. primal step from r and its halo; own u -> LDS;          barrier
+//   4. send the faces of u, receive the neighbours'.           barrier
+// With two voxels per thread the first is one of the tile's interior and the
+// second one of its surface (512 and 488 voxels of a 10^3 tile): the interior
+// half of steps 1 and 3 needs no halo and runs between sending and receiving.
+// Each voxel is updated with the marching sweep's operations in its order
+// (k_sweep), so the results are the same bits.
+//
+// Exchange.  A face value travels as one 8-byte entry (sequence << 32 | bits),
+// which carries its own arrival flag: no fence, one trip per exchange.
+// Measured on gfx950 with 500 work-groups and 192 entries each: 1.2 us per
+// exchange, against 2.5 us for data followed by a flag (a wait for the stores,
+// then a second trip) and 35-70 us with agent-scope release / acquire fences
+// (each writes back or invalidates an XCD's whole L2).  The entries are
+// relaxed agent-scope atomics, which pass the L2s by: with 1800 entries per
+// work-group, all 512 at once take 4.4 us, their traffic being the limit.
+// (Leaving the entries between work-groups of one XCD in its L2 takes 1.8 us
+// by itself, but the iteration of 80^3 stayed at 8.2-8.3 us.)  One entry per
+// value and direction is enough: a tile overwrites its u entries of iteration
+// n only after it has received the neighbour's r of iteration n + 1, which
+// that neighbour sends after consuming them (and the same with u and r
+// exchanged).  Sequence numbers never repeat: they start from an epoch that
+// the last work-group of each launch advances.
+//
+// Progress.  The waits need an instance's work-groups resident together, so a
+// launch holds no more work-groups than the device does (kBlkCapacity), and
+// the host keeps launches of different streams apart unless they fit beside
+// each other (wait_turn).  More groups than fit in one launch would not do:
+// the XCDs, and the shader engines within one, start their shares of a launch
+// at their own pace, and with 4 x 512 work-groups in one launch some that
+// waited kept out the ones they waited for.  No wait relies on any of this,
+// though: each is bounded by wait_ticks of the constant-rate clock.  Nothing is
+// written to the state before all of a group's work-groups have finished
+// (kCommit).  One that gives up before that decides the opposite (kRedo): all
+// of them leave, and the last redoes the instance's K iterations alone from
+// the untouched input state (slow, the same bits), and tells the host, which
+// goes back to the marching sweep (another process may hold part of the
+// device).
+//
+// Measured against the marching sweep, microseconds per iteration: one 80^3
+// 8.1 for 24.0 at K = 300 and 10.5 for 24.7 at K = 50 (the launch's fixed part
+// counts); at K = 50 four 80^3 39 for 79, one 40^3 4.5 for 10.0, 34 of them 44
+// for 76, one 20^3 4.0 for 7.7, 68 of them 15.3 for 30.7.
+#pragma once
+
+namespace svs {
+
+constexpr int kBlkThreads = 512;
+constexpr int kBlkCapacity = 512;       // work-groups the device holds at once: 2 on each of 256 CUs
+
+// Per V voxels per thread: LDS words of one u component with its halo and of
+// one r component with the halo along its axis, and chunks of 64 exchange
+// entries per wave.  For V = 2, 76 KiB of LDS: two work-groups per CU.
+template <int V> struct BlkCap;
+template <> struct BlkCap<1> { static constexpr int U = 1152, R = 768, H = 3; };
+template <> struct BlkCap<2> { static constexpr int U = 2048, R = 1440, H = 4; };
+// (one more word takes what nobody reads)
+template <int V> constexpr size_t blk_lds_bytes() { return sizeof(float) * (3 * BlkCap<V>::U + 9 * BlkCap<V>::R + 1); }
+constexpr int kBlkWaves = kBlkThreads / 64;
+// Chunks of one face: 3 components of A voxels in whole waves.
+__host__ __device__ constexpr int blk_chunks(int A) { return (3 * A + 63) / 64; }
+
+// One instance of a launch.
+struct alignas(16) BlockGroup {
+  int inst;         // index into the level's descriptor table
+  int first;        // its first work-group of the launch
+  int ntx, nty, ntz;
+  int tx, ty, tz;   // tile extent (the last one of a row may be shorter)
+  unsigned box;     // its first entry in the exchange buffer
+  int pad[3];
+};
+
+// One work-group of a launch: its group, its tile, and the work-groups of the
+// tile's neighbours across x-, x+, y-, y+, z-, z+ (-1: a face of the volume).
+// The host deals the tiles so that each XCD gets a compact piece of the
+// instance: rows of the state then share cache lines within one L2.
+struct alignas(16) BlockTile {
+  short group, bx, by, bz;
+  short nb[6];
+  short pad[6];
+};
+
+// One per plan, in the workspace, zero before the plan's first launch.
+struct alignas(16) BlockCtl {
+  unsigned ended;   // groups of the running launch that have left
+  unsigned epoch;   // launches so far
+  unsigned redone;  // instances redone by one work-group since the plan was created
+  unsigned pad;
+};
+// Per group of a launch, zero between launches.
+struct alignas(16) BlockDone {
+  unsigned arrived;  // work-groups that finished their iterations
+  unsigned left;     // work-groups that are through
+  unsigned verdict;  // kCommit or kRedo once decided
+  unsigned pad;
+};
+constexpr unsigned kCommit = 1, kRedo = 2;
+
+typedef unsigned long long u64;
+__device__ __forceinline__ void blk_send(u64* p, unsigned seq, float v) {
+  __hip_atomic_store(p, ((u64)seq << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 blk_peek(const u64* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned blk_add(unsigned* p, unsigned v) {
+  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned blk_get(const unsigned* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void blk_put(unsigned* p, unsigned v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Decides an undecided group; returns the verdict that holds.
+__device__ __forceinline__ unsigned blk_decide(unsigned* verdict, unsigned wanted) {
+  unsigned held = 0;
+  return __hip_atomic_compare_exchange_strong(verdict, &held, wanted, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT)
+             ? wanted
+             : held;
+}
+
+// Face tests of a position i of N along axis e, as bits of a mask.
+template <int BC>
+__device__ __forceinline__ unsigned face_bits(int i, int N, int e) {
+  unsigned m = 0;
+  if (BC == BD_MIRROR) {
+    m |= (i > 0 && i < N - 1) ? 1u : 0u;
+    m |= i > 1 ? 8u : 0u;
+    m |= i < N - 2 ? 64u : 0u;
+  } else {
+    m |= i > 0 ? 1u : 0u;
+    m |= i < N - 1 ? 8u : 0u;
+  }
+  return m << e;
+}
+constexpr int kFaceBits = 9;
+// v where bit b of m is set, else +0, by masking (cheaper than a compare and a
+// select per value).  For the adjoint this can turn a -0 term into +0, which
+// only a sum of zeros would show, as the sign of a zero.
+__device__ __forceinline__ float kept(float v, unsigned m, int b) {
+  return __uint_as_float(__float_as_uint(v) & (unsigned)((int)(m << (31 - b)) >> 31));
+}
+template <int BC>
+__device__ __forceinline__ float cd_fwd_sel(float bm, float b0, float bp, unsigned m, int e, float h) {
+  if (BC == BD_MIRROR) return kept((0.5f * (bp - bm)) / h, m, e);
+  const float lo = (m & (1u << e)) ? bm : b0, hi = (m & (8u << e)) ? bp : b0;
+  return (0.5f * (hi - lo)) / h;
+}
+template <int BC>
+__device__ __forceinline__ float cd_adj_sel(float pm, float p0, float pp, unsigned m, int e) {
+  if (BC == BD_MIRROR) return 0.5f * (kept(pm, m, 3 + e) - kept(pp, m, 6 + e));
+  return 0.5f * (((m & (1u << e)) ? pm : -p0) - ((m & (8u << e)) ? pp : -p0));
+}
+
+// The place in its tile of a thread's voxel j; x >= tx where it has none.
+// Both halves of V = 2 need tile edges of 3 or more (block_shape).
+template <int V>
+__device__ __forceinline__ void blk_voxel(int j, int t, int tx, int ty, int tz, int& x, int& y, int& z) {
+  if (V == 1) {
+    x = t % tx; t /= tx;
+    y = t % ty; z = t / ty;
+  } else if (j == 0) {  // interior
+    const int ix = tx - 2, iy = ty - 2;
+    x = 1 + t % ix; t /= ix;
+    y = 1 + t % iy; z = 1 + t / iy;
+    if (z >= tz - 1) x = tx;
+  } else {  // surface: the two z faces, then the rim of every plane between
+    const int face = tx * ty, rim = 2 * (tx + ty - 2);
+    if (t < 2 * face) {
+      z = t < face ? 0 : tz - 1;
+      t -= t < face ? 0 : face;
+      x = t % tx; y = t / tx;
+    } else {
+      t -= 2 * face;
+      z = 1 + t / rim;
+      t %= rim;
+      if (t < 2 * tx) {
+        y = t < tx ? 0 : ty - 1;
+        x = t < tx ? t : t - tx;
+      } else {
+        t -= 2 * tx;
+        x = (t & 1) ? tx - 1 : 0;
+        y = 1 + (t >> 1);
+      }
+      if (z >= tz - 1) x = tx;
+    }
+  }
+}
+
+__device__ __forceinline__ u64* blk_entry(u64* base, unsigned byte) {
+  return reinterpret_cast<u64*>(reinterpret_cast<char*>(base) + byte);
+}
+__device__ __forceinline__ float* blk_at(float* lds, unsigned byte) {
+  return reinterpret_cast<float*>(reinterpret_cast<char*>(lds) + byte);
+}
+// D q or, without anisotropy, q itself.
+template <bool ANISO>
+__device__ __forceinline__ void apply_tensor(float s, const float n[3], const float t1[3], const float q[3],
+                                             float out[3]) {
+  if (ANISO) aniso_row(s, n, t1, q, out);
+  else { out[0] = q[0]; out[1] = q[1]; out[2] = q[2]; }
+}
+
+// The dual prox of a voxel's three rows (prox_dual_row, and zero when wtv is,
+// tvl13d.py:223-224).  ball.y = recip_nr(wtv) and ball.most the largest squared
+// norm for which the short division and square root hold (negative: never);
+// a voxel with a value outside their range takes the plain operations.  Below
+// the range of sqrt_nr the norm is far inside the ball and den is 1 either
+// way (its NaN for 0 included: fmaxf returns 1).
+struct Ball {
+  float wtv, y, most;
+};
+__device__ __forceinline__ Ball make_ball(float wtv) {
+  Ball b{wtv, 0.0f, -1.0f};
+  if (wtv >= 0x1p-40f && wtv <= 0x1p40f) {
+    const float r = 0x1p20f * wtv;  // den stays within 2^20
+    b.y = recip_nr(wtv);
+    b.most = fminf(r * r, 0x1p100f);
+  }
+  return b;
+}
+__device__ __forceinline__ void prox_dual(float (&p)[9], const Ball& ball) {
+  float ns[3], least = fabsf(p[0]), most;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    ns[c] = p[3 * c] * p[3 * c];
+    ns[c] += p[3 * c + 1] * p[3 * c + 1];
+    ns[c] += p[3 * c + 2] * p[3 * c + 2];
+  }
+#pragma unroll
+  for (int e = 1; e < 9; ++e) least = fminf(least, fabsf(p[e]));
+  most = fmaxf(fmaxf(ns[0], ns[1]), ns[2]);
+  if (least >= 0x1p-100f && most <= ball.most) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const float den = fmaxf(1.0f, div_nr(sqrt_nr(ns[c]), ball.wtv, ball.y));
+      const float y = recip_nr(den);
+#pragma unroll
+      for (int e = 0; e < 3; ++e) p[3 * c + e] = div_nr(p[3 * c + e], den, y);
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const float den = fmaxf(1.0f, sqrtf(ns[c]) / ball.wtv);
+#pragma unroll
+      for (int e = 0; e < 3; ++e) p[3 * c + e] = ball.wtv == 0.0f ? 0.0f : p[3 * c + e] / den;
+    }
+  }
+}
+
+// What the data term's prox needs of a voxel for a whole warp: |g|^2 and its
+// recip_nr; y is 0 where the reference's |g|^2 > 1e-10 fails (no step inside
+// the band), negative where the short division does not hold.
+struct DataTerm {
+  float g2, y;
+};
+__device__ __forceinline__ DataTerm make_data_term(const float rg[4]) {
+  DataTerm t;
+  t.g2 = rg[1] * rg[1];
+  t.g2 += rg[2] * rg[2];
+  t.g2 += rg[3] * rg[3];
+  t.y = (double)t.g2 > 1e-10 ? (t.g2 <= 0x1p20f ? recip_nr(t.g2) : -1.0f) : 0.0f;
+  return t;
+}
+
+// u^{n+1} of one voxel from its adjoint terms a[c][e] (before the division by
+// h): prox_primal_point at u - tau div with rho at u.
+__device__ __forceinline__ void primal_point(float u[3], const float (&a)[3][3], float hX, float hY, float hZ,
+                                             const float rg[4], const DataTerm& dt, float tau, float factor) {
+  const float g[3] = {rg[1], rg[2], rg[3]};
+  const float sm = (u[0] * g[0] + u[2] * g[2]) + u[1] * g[1];  // (a + c) + b, as torch's sum
+  const float rho = rg[0] + sm;
+  const float band = factor * dt.g2;
+  const bool below = rho < -band, above = rho > band;
+  float delta[3];
+  if (below || above) {
+    const float f = below ? factor : -factor;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) delta[c] = f * g[c];
+  } else if (dt.y != 0.0f) {
+    float num[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) num[c] = -rho * g[c];
+    const float least = fminf(fminf(fabsf(num[0]), fabsf(num[1])), fabsf(num[2]));
+    const float most = fmaxf(fmaxf(fabsf(num[0]), fabsf(num[1])), fabsf(num[2]));
+    if (dt.y > 0.0f && least >= 0x1p-100f && most <= 0x1p60f) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) delta[c] = div_nr(num[c], dt.g2, dt.y);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) delta[c] = num[c] / dt.g2;
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) delta[c] = 0.0f;
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const float div = a[c][0] / hX + a[c][1] / hY + a[c][2] / hZ;
+    const float step = tau * div;
+    const float v = u[c] - step;
+    u[c] = v + delta[c];
+  }
+}
+
+// The K iterations of one instance by one work-group through global memory,
+// from buffer `parity` (which it overwrites on the way) into parity ^ 1.
+template <int BC, bool ANISO>
+__device__ __forceinline__ void redo_instance(const LevelDesc& d, const float* __restrict__ sched, int K, int parity,
+                                              const Ball& ball) {
+  const int NZ = d.NZ, NY = d.NY, NX = d.NX, PL = NY * NX, N = (int)d.N;
+  const float hZ = d.hZ, hY = d.hY, hX = d.hX;
+  for (int it = 0; it < K; ++it) {
+    const float* u = d.u[parity ^ (it & 1)];
+    const float* p = d.p[parity ^ (it & 1)];
+    float* un = d.u[parity ^ 1 ^ (it & 1)];
+    float* pn = d.p[parity ^ 1 ^ (it & 1)];
+    for (int v = threadIdx.x; v < N; v += kBlkThreads) {
+      const int x = v % NX, y = (v / NX) % NY, z = v / PL;
+      const int xm = x > 0 ? v - 1 : v, xp = x < NX - 1 ? v + 1 : v;
+      const int ym = y > 0 ? v - NX : v, yp = y < NY - 1 ? v + NX : v;
+      const int zm = z > 0 ? v - PL : v, zp = z < NZ - 1 ? v + PL : v;
+      float s = 0.0f, n[3] = {0.0f, 0.0f, 0.0f}, t1[3] = {0.0f, 0.0f, 0.0f};
+      if (ANISO) {
+        const float4 a = d.SN[v];
+        s = a.x; n[0] = a.y; n[1] = a.z; n[2] = a.w;
+        tangent1(n, t1);
+      }
+      float pv[9];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float* uc = u + (int64_t)c * N;
+        const float q[3] = {cd_fwd(uc[xm], uc[v], uc[xp], x, NX, hX, BC), cd_fwd(uc[ym], uc[v], uc[yp], y, NY, hY, BC),
+                            cd_fwd(uc[zm], uc[v], uc[zp], z, NZ, hZ, BC)};
+        float dq[3];
+        apply_tensor<ANISO>(s, n, t1, q, dq);
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          const float inc = sched[4 * it] * dq[e];
+          pv[3 * c + e] = p[(int64_t)(3 * c + e) * N + v] + inc;
+        }
+      }
+      prox_dual(pv, ball);
+#pragma unroll
+      for (int e = 0; e < 9; ++e) pn[(int64_t)e * N + v] = pv[e];
+    }
+    __syncthreads();
+    // (D p')_{c,e} at voxel v, recomputed from p'.
+    auto r_at = [&](int c, int e, int v) __attribute__((always_inline)) {
+      const float q[3] = {pn[(int64_t)(3 * c) * N + v], pn[(int64_t)(3 * c + 1) * N + v],
+                          pn[(int64_t)(3 * c + 2) * N + v]};
+      if (!ANISO) return e == 0 ? q[0] : e == 1 ? q[1] : q[2];
+      const float4 a = d.SN[v];
+      const float n[3] = {a.y, a.z, a.w};
+      float t1[3], rr[3];
+      tangent1(n, t1);
+      aniso_row(a.x, n, t1, q, rr);
+      return e == 0 ? rr[0] : e == 1 ? rr[1] : rr[2];
+    };
+    for (int v = threadIdx.x; v < N; v += kBlkThreads) {
+      const int x = v % NX, y = (v / NX) % NY, z = v / PL;
+      const int lo[3] = {x > 0 ? v - 1 : v, y > 0 ? v - NX : v, z > 0 ? v - PL : v};
+      const int hi[3] = {x < NX - 1 ? v + 1 : v, y < NY - 1 ? v + NX : v, z < NZ - 1 ? v + PL : v};
+      const int pos[3] = {x, y, z}, size[3] = {NX, NY, NZ};
+      float a[3][3], uv[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        uv[c] = u[(int64_t)c * N + v];
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          a[c][e] = cd_adj(r_at(c, e, lo[e]), r_at(c, e, v), r_at(c, e, hi[e]), pos[e], size[e], BC);
+      }
+      const float4 b = d.RG[v];
+      const float rg[4] = {b.x, b.y, b.z, b.w};
+      primal_point(uv, a, hX, hY, hZ, rg, make_data_term(rg), sched[4 * it + 1], sched[4 * it + 2]);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) un[(int64_t)c * N + v] = uv[c];
+    }
+    __syncthreads();
+  }
+  if (!(K & 1)) {  // an even count ends where it began
+    for (int v = threadIdx.x; v < N; v += kBlkThreads) {
+      for (int c = 0; c < 3; ++c) d.u[parity ^ 1][(int64_t)c * N + v] = d.u[parity][(int64_t)c * N + v];
+      for (int e = 0; e < 9; ++e) d.p[parity ^ 1][(int64_t)e * N + v] = d.p[parity][(int64_t)e * N + v];
+    }
+  }
+}
+
+// K iterations (schedule positions 0 .. K-1) of the launch's instances, from
+// buffer `parity` into buffer parity ^ 1; one work-group per tile.
+template <int BC, bool ANISO, bool UNIT_H, int V>
+__global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_sweep_block(
+    const LevelDesc* __restrict__ descs, const BlockGroup* __restrict__ groups,
+    const BlockTile* __restrict__ tiles, int ngroups, const float* __restrict__ sched, int K, int parity, float wtv,
+    u64* __restrict__ box, BlockCtl* __restrict__ ctl, BlockDone* __restrict__ done, u64 wait_ticks,
+    unsigned* __restrict__ redone) {
+  constexpr int UC = BlkCap<V>::U, RC = BlkCap<V>::R, H = BlkCap<V>::H;
+  extern __shared__ float lds[];
+  float* U = lds;           // [3][UC]
+  float* R = lds + 3 * UC;  // [9][RC]: r[3c + e] with a halo along axis e
+  __shared__ unsigned sh_epoch;
+  __shared__ unsigned sh_verdict;
+  __shared__ int sh_dead, sh_last;
+  const int tid = threadIdx.x;
+  if (tid == 0) {
+    sh_epoch = __hip_atomic_load(&ctl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sh_dead = 0;
+  }
+  __syncthreads();
+  const unsigned seq0 = (unsigned)__builtin_amdgcn_readfirstlane((int)sh_epoch) * (2u * (unsigned)K + 2u) + 1u;
+  const BlockTile T = tiles[blockIdx.x];
+  const int gi = T.group;
+  const BlockGroup G = groups[gi];
+  const LevelDesc& d = descs[G.inst];
+  const int NZ = d.NZ, NY = d.NY, NX = d.NX;
+  const int64_t N = d.N;
+  const float hZ = UNIT_H ? 1.0f : d.hZ, hY = UNIT_H ? 1.0f : d.hY, hX = UNIT_H ? 1.0f : d.hX;
+  const int slot = (int)blockIdx.x - G.first;
+  const int tx = G.tx, ty = G.ty, tz = G.tz;
+  const int x0 = T.bx * tx, y0 = T.by * ty, z0 = T.bz * tz;
+  const int nx = min(tx, NX - x0), ny = min(ty, NY - y0), nz = min(tz, NZ - z0);
+  const int ux = tx + 2, uxy = ux * (ty + 2);
+
+  // ---- this thread's voxels and their state
+  const float* uin = d.u[parity];
+  const float* pin = d.p[parity];
+  float u[V][3], p[V][9], sn[V][4], rg[V][4];
+  // Own cell in U and in the three kinds of r component as pairs of 16-bit
+  // numbers, and the face tests as bits (registers are what V = 2 lacks).
+  unsigned cell_ux[V], cell_yz[V], faces = 0;
+  DataTerm dt[V];
+  bool own[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    int x, y, z;
+    blk_voxel<V>(j, tid, tx, ty, tz, x, y, z);
+    own[j] = x < nx && y < ny && z < nz;
+    faces |= (face_bits<BC>(x0 + x, NX, 0) | face_bits<BC>(y0 + y, NY, 1) | face_bits<BC>(z0 + z, NZ, 2))
+             << (kFaceBits * j);
+    const int ui = (x + 1) + ux * (y + 1) + uxy * (z + 1);
+    cell_ux[j] = own[j] ? (unsigned)(ui | (((x + 1) + ux * (y + ty * z)) << 16)) : 0u;
+    cell_yz[j] = own[j] ? (unsigned)((x + tx * ((y + 1) + (ty + 2) * z)) | ((x + tx * (y + ty * (z + 1))) << 16)) : 0u;
+    const int64_t i = own[j] ? ((int64_t)(z0 + z) * NY + (y0 + y)) * NX + (x0 + x) : 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      u[j][c] = uin[c * N + i];
+      if (own[j]) U[c * UC + ui] = u[j][c];
+    }
+#pragma unroll
+    for (int e = 0; e < 9; ++e) p[j][e] = pin[e * N + i];
+    const float4 a = ANISO ? d.SN[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float4 b = d.RG[i];
+    sn[j][0] = a.x; sn[j][1] = a.y; sn[j][2] = a.z; sn[j][3] = a.w;
+    rg[j][0] = b.x; rg[j][1] = b.y; rg[j][2] = b.z; rg[j][3] = b.w;
+    dt[j] = make_data_term(rg[j]);
+  }
+  const Ball ball = make_ball(wtv);
+
+  // ---- exchange entries.  A tile's entries are cut into chunks of 64, one
+  // wave's worth, each of a single face (x-, x+, y-, y+, z-, z+ in order; entry
+  // i of a face is component i / A of voxel i % A): the neighbour, its entries'
+  // place are the same for a whole wave, and lanes without a voxel
+  // send and receive something nobody reads.  The neighbour across a face reads
+  // what this tile sends as what arrives over its opposite face.
+  const int area[3] = {ty * tz, tx * tz, tx * ty};
+  const int nch[3] = {blk_chunks(area[0]), blk_chunks(area[1]), blk_chunks(area[2])};
+  const int chunks = 2 * (nch[0] + nch[1] + nch[2]);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  constexpr unsigned kTrash = (3 * UC + 9 * RC) * 4;
+  unsigned usrc[H], udst[H], rsrc[H], rdst[H];  // LDS bytes: boundary cell sent, halo cell filled
+  unsigned from[H];   // the neighbour's u entries of chunk k, counted from box
+  unsigned has = 0;   // chunk k has a neighbour
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    usrc[k] = rsrc[k] = 0;
+    udst[k] = rdst[k] = kTrash;
+    from[k] = 0;
+    const int ch = wave + k * kBlkWaves;
+    int axis = 0, r = ch;
+    if (r >= 2 * nch[0]) { r -= 2 * nch[0]; axis = 1; }
+    if (axis == 1 && r >= 2 * nch[1]) { r -= 2 * nch[1]; axis = 2; }
+    const int up = r >= nch[axis] ? 1 : 0;
+    r -= up * nch[axis];
+    const int there = axis == 0 ? (up ? T.nb[1] : T.nb[0]) : axis == 1 ? (up ? T.nb[3] : T.nb[2])
+                                                                      : (up ? T.nb[5] : T.nb[4]);
+    if (ch >= chunks || there < 0) continue;
+    has |= 1u << k;
+    from[k] = G.box + (unsigned)((there - G.first) * 2 * chunks + (up ? ch - nch[axis] : ch + nch[axis])) * 64u;
+    const int A = area[axis], i = r * 64 + lane;
+    const int c = i / A, v = i - c * A;
+    const int w = axis == 0 ? ty : tx;
+    const int a = v % w, b = v / w;
+    int x = a, y = b, z = b, hx, hy, hz;
+    if (axis == 0) {
+      y = a; x = up ? nx - 1 : 0;
+      hx = up ? nx : -1; hy = y; hz = z;
+    } else if (axis == 1) {
+      y = up ? ny - 1 : 0;
+      hx = x; hy = up ? ny : -1; hz = z;
+    } else {
+      z = up ? nz - 1 : 0;
+      hx = x; hy = y; hz = up ? nz : -1;
+    }
+    if (i >= 3 * A || x >= nx || y >= ny || z >= nz) continue;
+    auto ucell = [&](int X, int Y, int Z) __attribute__((always_inline)) {
+      return 4u * (unsigned)(c * UC + (X + 1) + ux * (Y + 1) + uxy * (Z + 1));
+    };
+    auto rcell = [&](int X, int Y, int Z) __attribute__((always_inline)) {
+      const int at = axis == 0 ? (X + 1) + ux * (Y + ty * Z)
+                               : axis == 1 ? X + tx * ((Y + 1) + (ty + 2) * Z) : X + tx * (Y + ty * (Z + 1));
+      return 4u * (unsigned)(3 * UC + (3 * c + axis) * RC + at);
+    };
+    usrc[k] = ucell(x, y, z);
+    udst[k] = ucell(hx, hy, hz);
+    rsrc[k] = rcell(x, y, z);
+    rdst[k] = rcell(hx, hy, hz);
+    // The first iteration's halo of u comes from the input state.
+    *blk_at(lds, udst[k]) = uin[c * N + ((int64_t)(z0 + hz) * NY + (y0 + hy)) * NX + (x0 + hx)];
+  }
+
+  // Opaque where it is used, so that an address stays a scalar base and this
+  // 32-bit offset: as hoisted 64-bit sums the addresses cost 32 registers, and
+  // formed in a register that a load in flight is to fill they made each load
+  // wait for the one before it (9.7 us per iteration of 80^3, 8.3 like this).
+  auto lane8 = [&]() __attribute__((always_inline)) {
+    unsigned at = 8u * (unsigned)lane;
+    asm volatile("" : "+v"(at));
+    return at;
+  };
+  // Sends this wave's boundary cells under `seq`; kind 0 is u, 1 is r.
+  auto send = [&](const unsigned(&src)[H], int kind, unsigned seq) __attribute__((always_inline)) {
+    u64* const mine = box + (G.box + (unsigned)(slot * 2 + kind) * (unsigned)chunks * 64u);
+    float edge[H];
+#pragma unroll
+    for (int k = 0; k < H; ++k) edge[k] = *blk_at(lds, src[k]);
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      if (!((has >> k) & 1u)) continue;
+      blk_send(blk_entry(mine + 64 * (wave + k * kBlkWaves), lane8()), seq, edge[k]);
+    }
+  };
+  // Fills this wave's halo cells with what arrives under `seq`.
+  auto receive = [&](const unsigned(&dst)[H], int kind, unsigned seq) __attribute__((always_inline)) {
+    unsigned todo = has;
+    u64 give_up = 0;
+    for (unsigned spins = 0; todo;) {
+      u64 e[H];
+      // All of them each time (without a neighbour: the buffer's first ones), so
+      // that they are in flight together: 8.1 us per iteration of 80^3, 8.3 with
+      // a branch around each.
+#pragma unroll
+      for (int k = 0; k < H; ++k) {
+        e[k] = blk_peek(blk_entry(box + (from[k] + (unsigned)kind * (unsigned)chunks * 64u), lane8()));
+      }
+#pragma unroll
+      for (int k = 0; k < H; ++k) {
+        if (!((todo >> k) & 1u)) continue;
+        if (__ballot((unsigned)(e[k] >> 32) != seq) == 0) {
+          *blk_at(lds, dst[k]) = __uint_as_float((unsigned)e[k]);
+          todo &= ~(1u << k);
+        }
+      }
+      if (todo && (++spins & 15u) == 0) {
+        const u64 now = wall_clock64();
+        if (give_up == 0) give_up = now + wait_ticks;
+        else if (now >= give_up || blk_get(&done[gi].verdict) == kRedo) {
+          sh_dead = 1;
+          break;
+        }
+      }
+    }
+  };
+
+  __syncthreads();
+  bool dead = sh_dead != 0;
+  for (int it = 0; it < K && !dead; ++it) {
+    const float sigma = sched[4 * it], tau = sched[4 * it + 1], factor = sched[4 * it + 2];
+    // Unpacked, and turned into addresses, each iteration: hoisted out of the
+    // loop the results would spill.
+    asm volatile("" : "+v"(faces));
+#pragma unroll
+    for (int j = 0; j < V; ++j) asm volatile("" : "+v"(cell_ux[j]), "+v"(cell_yz[j]));
+    const unsigned seq = seq0 + 2u * (unsigned)it;
+    // ---- dual step of voxel j
+    auto dual = [&](int j) __attribute__((always_inline)) {
+      if (!own[j]) return;
+      const unsigned m = faces >> (kFaceBits * j);
+      const float* Ui = U + (cell_ux[j] & 0xffffu);
+      const int ri[3] = {(int)(cell_ux[j] >> 16), (int)(cell_yz[j] & 0xffffu), (int)(cell_yz[j] >> 16)};
+      // The neighbours' loads run one row ahead of their use.  A halo cell past
+      // a volume face is never written; its value is not selected.
+      float b[3][6];
+      auto load = [&](int c) __attribute__((always_inline)) {
+        const float* Uc = Ui + c * UC;
+        b[c][0] = Uc[-1]; b[c][1] = Uc[1];
+        b[c][2] = Uc[-ux]; b[c][3] = Uc[ux];
+        b[c][4] = Uc[-uxy]; b[c][5] = Uc[uxy];
+      };
+      load(0);
+      float t1[3] = {0.0f, 0.0f, 0.0f};
+      const float n[3] = {sn[j][1], sn[j][2], sn[j][3]};
+      if (ANISO) tangent1(n, t1);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        if (c < 2) load(c + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const float q[3] = {cd_fwd_sel<BC>(b[c][0], u[j][c], b[c][1], m, 0, hX),
+                            cd_fwd_sel<BC>(b[c][2], u[j][c], b[c][3], m, 1, hY),
+                            cd_fwd_sel<BC>(b[c][4], u[j][c], b[c][5], m, 2, hZ)};
+        float dq[3];
+        apply_tensor<ANISO>(sn[j][0], n, t1, q, dq);
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          const float inc = sigma * dq[e];
+          p[j][3 * c + e] = p[j][3 * c + e] + inc;
+        }
+      }
+      prox_dual(p[j], ball);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float pv[3] = {p[j][3 * c], p[j][3 * c + 1], p[j][3 * c + 2]};
+        float rr[3];
+        apply_tensor<ANISO>(sn[j][0], n, t1, pv, rr);
+#pragma unroll
+        for (int e = 0; e < 3; ++e) R[(3 * c + e) * RC + ri[e]] = rr[e];
+      }
+    };
+    // ---- primal step of voxel j
+    auto primal = [&](int j) __attribute__((always_inline)) {
+      if (!own[j]) return;
+      const int ri[3] = {(int)(cell_ux[j] >> 16), (int)(cell_yz[j] & 0xffffu), (int)(cell_yz[j] >> 16)};
+      const int step[3] = {1, tx, tx * ty};
+      const unsigned m = faces >> (kFaceBits * j);
+      float lo[3][3], hi[3][3], mid[3][3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          const float* Re = R + (3 * c + e) * RC + ri[e];
+          lo[c][e] = Re[-step[e]];
+          hi[c][e] = Re[step[e]];
+          mid[c][e] = BC == BD_MIRROR ? 0.0f : Re[0];
+        }
+      float a[3][3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int e = 0; e < 3; ++e) a[c][e] = cd_adj_sel<BC>(lo[c][e], mid[c][e], hi[c][e], m, e);
+      primal_point(u[j], a, hX, hY, hZ, rg[j], dt[j], tau, factor);
+      float* Ui = U + (cell_ux[j] & 0xffffu);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) Ui[c * UC] = u[j][c];
+    };
+    if (V == 2) dual(0);
+    if (it > 0) {
+      receive(udst, 0, seq - 1u);
+      __syncthreads();
+      if (sh_dead) { dead = true; break; }
+    }
+    dual(V - 1);
+    __syncthreads();
+    send(rsrc, 1, seq);
+    if (V == 2) primal(0);
+    receive(rdst, 1, seq);
+    __syncthreads();
+    if (sh_dead) { dead = true; break; }
+    primal(V - 1);
+    if (it + 1 == K) break;
+    __syncthreads();
+    send(usrc, 0, seq + 1u);
+  }
+  // ---- commit or redo, alike in all work-groups of the group.
+  const unsigned ntiles = (unsigned)(G.ntx * G.nty * G.ntz);
+  if (tid == 0) {
+    unsigned v = 0;
+    if (dead) v = blk_decide(&done[gi].verdict, kRedo);
+    else if (blk_add(&done[gi].arrived, 1u) + 1u == ntiles) v = blk_decide(&done[gi].verdict, kCommit);
+    for (u64 give_up = wall_clock64() + wait_ticks; v == 0;) {
+      v = blk_get(&done[gi].verdict);
+      if (v == 0 && wall_clock64() >= give_up) v = blk_decide(&done[gi].verdict, kRedo);
+    }
+    sh_verdict = v;
+  }
+  __syncthreads();
+  const unsigned verdict = (unsigned)__builtin_amdgcn_readfirstlane((int)sh_verdict);
+  if (verdict == kCommit) {
+    float* uout = d.u[parity ^ 1];
+    float* pout = d.p[parity ^ 1];
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+      if (own[j]) {
+        int x, y, z;
+        blk_voxel<V>(j, tid, tx, ty, tz, x, y, z);
+        const int64_t i = ((int64_t)(z0 + z) * NY + (y0 + y)) * NX + (x0 + x);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) uout[c * N + i] = u[j][c];
+#pragma unroll
+        for (int e = 0; e < 9; ++e) pout[e * N + i] = p[j][e];
+      }
+  }
+  // ---- leave
+  if (tid == 0) sh_last = blk_add(&done[gi].left, 1u) + 1u == ntiles;
+  __syncthreads();
+  if (!sh_last) return;
+  if (verdict == kRedo) {
+    if (tid == 0) {
+      blk_add(&ctl->redone, 1u);
+      __hip_atomic_store(redone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    redo_instance<BC, ANISO>(d, sched, K, parity, ball);
+  }
+  if (tid == 0) {
+    blk_put(&done[gi].arrived, 0u);
+    blk_put(&done[gi].left, 0u);
+    blk_put(&done[gi].verdict, 0u);
+    if (blk_add(&ctl->ended, 1u) + 1u == (unsigned)ngroups) {  // the launch has no other work-group left
+      blk_put(&ctl->ended, 0u);
+      blk_add(&ctl->epoch, 1u);
+    }
+  }
+}
+
+}  // namespace svs

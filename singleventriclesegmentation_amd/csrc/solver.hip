@@ -61,6 +61,12 @@ struct alignas(16) LevelDesc {
 constexpr int kBlock = 256;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, work-groups dealt round-robin
 
+}  // namespace svs
+
+#include "block_sweep.hpp"
+
+namespace svs {
+
 // Taps in flight per tricubic gather (the LOOP level of sample_cubic_impl)
 // for the per-warp linearisation, the restriction and the prolongation.
 // Level 1 (one z-plane of taps at a time) takes the linearisation from 233
@@ -909,6 +915,22 @@ __global__ __launch_bounds__(1024) void k_sweep_resident(const LevelDesc* __rest
     }
 }
 
+// Exchanges the two halves of the ping-pong state of the listed instances: the
+// marching sweep leaves an even number of iterations where it began, the
+// block-resident sweep always in the other half, and a level that runs both
+// goes on from one parity.
+__global__ __launch_bounds__(64) void k_swap_state(LevelDesc* __restrict__ descs, const int* __restrict__ list, int n) {
+  const int k = (int)(blockIdx.x * 64 + threadIdx.x);
+  if (k >= n) return;
+  LevelDesc& d = descs[list[k]];
+  float* u = d.u[0];
+  float* p = d.p[0];
+  d.u[0] = d.u[1];
+  d.p[0] = d.p[1];
+  d.u[1] = u;
+  d.p[1] = p;
+}
+
 // --------------------------------------------------- iteration statistics
 // Per-iteration statistics of every instance from the sweeps' partial sums,
 // part[(n * ngroups + g) * wpg + w] = (sum (u' - u)^2, sum (p' - p)^2,
@@ -969,6 +991,24 @@ struct LevelPlan {
   int res_capable = 0;           // voxels per thread the level would need (0: too large)
   int res_threads = 0;
   size_t res_lds = 0;
+  // Block-resident sweep (k_sweep_block): voxels per thread, the instances it
+  // runs as groups of tiles split over launches, and whether the level uses
+  // it.  rest: the instances it does not hold, with a tile table of their own.
+  int blk_v = 0;
+  bool blk_capable = false;
+  bool blk_on = false;
+  struct BlockLaunch {
+    int first, ngroups, tiles;
+  };
+  std::vector<BlockGroup> blk_groups;
+  std::vector<BlockLaunch> blk_launches;
+  std::vector<BlockTile> blk_tiles;  // launch after launch
+  BlockGroup* blk_dev = nullptr;
+  BlockTile* blk_tiles_dev = nullptr;
+  std::vector<int> rest;
+  int* rest_dev = nullptr;
+  SweepTile* rest_tiles = nullptr;
+  int nrest_tiles = 0;
 };
 
 }  // namespace svs
@@ -1007,6 +1047,17 @@ struct svs_plan {
   float* stats_out = nullptr;
   float4* stats_part = nullptr;
   size_t stats_part_bytes = 0;
+  // Block-resident sweeps: the exchange buffer and counters (in the
+  // workspace), the longest wait for a neighbour, and the work-groups that run
+  // at once in the largest launch.
+  svs::u64* blk_box = nullptr;
+  size_t blk_box_bytes = 0;
+  svs::BlockCtl* blk_ctl = nullptr;
+  svs::BlockDone* blk_done = nullptr;
+  unsigned long long blk_wait_ticks = 20000000ull;  // 0.2 s of the 100 MHz clock
+  unsigned* blk_redone = nullptr;  // pinned (behind staging): the device had to redo an instance
+  int blk_need = 0;
+  int device = 0;
 };
 
 namespace svs {
@@ -1137,6 +1188,7 @@ static std::vector<int> cz_candidates(const LevelPlan& L) {
 static std::mutex g_tune_mu;
 static std::map<std::string, SweepShape> g_tuned;
 static std::map<std::string, bool> g_tuned_resident;  // levels that qualify: resident faster?
+static std::map<std::string, bool> g_tuned_blocks;    // the same for the block-resident sweep
 
 static std::string tune_key(const svs_tvl1_params& P, const LevelPlan& L) {
   std::map<std::array<int, 3>, int> hist;
@@ -1194,6 +1246,187 @@ static void choose_sweep_shape(const svs_tvl1_params& P, LevelPlan& L, int ninst
   L.bx = bx; L.by = by; L.cz = cz;
 }
 
+// Tile extent of one instance for the block-resident sweep, or false when it
+// needs more work-groups than the device holds.  Costs in ns per tile and
+// iteration on a loaded chip: about 1.9 per voxel (both half-steps) and 1 per
+// exchange entry.  `spread`: every tile of the launch runs at once, so the
+// largest tile counts; otherwise all tiles share the chip and their sum does.
+template <int V>
+static bool block_shape(const LevelDesc& d, bool spread, BlockGroup* g) {
+  double best = 0.0;
+  auto pieces = [](int n, int k) { return (n + k - 1) / k; };
+  int last_x = 0;
+  for (int ntx = pieces(d.NX, V * kBlkThreads); ntx <= std::min(d.NX, kBlkCapacity); ++ntx) {
+    const int tx = pieces(d.NX, ntx);
+    if (tx == last_x) continue;
+    last_x = tx;
+    int last_y = 0;
+    for (int nty = pieces(d.NY, V * kBlkThreads / tx); nty <= std::min(d.NY, kBlkCapacity / pieces(d.NX, tx)); ++nty) {
+      const int ty = pieces(d.NY, nty);
+      if (ty == last_y) continue;
+      last_y = ty;
+      int last_z = 0;
+      const int cx = pieces(d.NX, tx), cy = pieces(d.NY, ty);
+      for (int ntz = pieces(d.NZ, V * kBlkThreads / (tx * ty)); ntz <= std::min(d.NZ, kBlkCapacity / (cx * cy)); ++ntz) {
+        const int tz = pieces(d.NZ, ntz);
+        if (tz == last_z) continue;
+        last_z = tz;
+        const int cz = pieces(d.NZ, tz);
+        const int64_t tiles = (int64_t)cx * cy * cz;
+        const int chunks = 2 * (blk_chunks(ty * tz) + blk_chunks(tx * tz) + blk_chunks(tx * ty)), S = 64 * chunks;
+        const int interior = (tx - 2) * (ty - 2) * (tz - 2);
+        if (V == 2 && (tx < 3 || ty < 3 || tz < 3 || interior > kBlkThreads ||
+                       tx * ty * tz - interior > kBlkThreads))
+          continue;
+        if (tiles > kBlkCapacity || chunks > BlkCap<V>::H * kBlkWaves ||
+            (tx + 2) * (ty + 2) * (tz + 2) > BlkCap<V>::U || (tx + 2) * ty * tz > BlkCap<V>::R ||
+            tx * (ty + 2) * tz > BlkCap<V>::R || tx * ty * (tz + 2) > BlkCap<V>::R)
+          continue;
+        const double cost = spread ? 1.9 * std::max(tx * ty * tz, 256) + 1.0 * std::max(S, 512) + 1e-3 * (double)tiles
+                                   : (1.9 * tx * ty * tz + 1.0 * S) * (double)tiles;
+        if (best == 0.0 || cost < best) {
+          best = cost;
+          g->ntx = cx; g->nty = cy; g->ntz = cz;
+          g->tx = tx; g->ty = ty; g->tz = tz;
+        }
+      }
+    }
+  }
+  return best > 0.0;
+}
+
+static bool block_shape_v(int v, const LevelDesc& d, bool spread, BlockGroup* g) {
+  return v == 1 ? block_shape<1>(d, spread, g) : block_shape<2>(d, spread, g);
+}
+
+static int block_tiles(const BlockGroup& g) { return g.ntx * g.nty * g.ntz; }
+static int block_entries(const BlockGroup& g) {  // of u and r, per tile
+  return 2 * 64 * 2 * (blk_chunks(g.ty * g.tz) + blk_chunks(g.tx * g.tz) + blk_chunks(g.tx * g.ty));
+}
+
+// Deals a group's tiles to its work-groups so that each XCD gets a compact
+// piece: work-group w runs on XCD w % 8, and the tiles (x fastest) are halved
+// along their longest side until each XCD has its share.  at[w - first] is
+// the tile of work-group w.
+static void deal_tiles(const BlockGroup& g, std::vector<int>& at) {
+  const int n = block_tiles(g);
+  std::vector<std::vector<int>> slots(kXcds);
+  for (int w = 0; w < n; ++w) slots[(g.first + w) % kXcds].push_back(w);
+  at.assign(n, 0);
+  auto pos = [&](int t, int axis) {
+    return axis == 0 ? t % g.ntx : axis == 1 ? (t / g.ntx) % g.nty : t / (g.ntx * g.nty);
+  };
+  struct Part {
+    std::vector<int> tiles;
+    int lo, hi;  // XCDs
+  };
+  std::vector<Part> todo(1);
+  for (int t = 0; t < n; ++t) todo[0].tiles.push_back(t);
+  todo[0].lo = 0;
+  todo[0].hi = kXcds;
+  while (!todo.empty()) {
+    Part p = std::move(todo.back());
+    todo.pop_back();
+    if (p.hi - p.lo == 1) {
+      for (size_t i = 0; i < p.tiles.size(); ++i) at[slots[p.lo][i]] = p.tiles[i];
+      continue;
+    }
+    int axis = 0, longest = -1;
+    for (int a = 2; a >= 0; --a) {  // ties: z before y before x, rows stay whole
+      int lo = 1 << 30, hi = -1;
+      for (int t : p.tiles) { lo = std::min(lo, pos(t, a)); hi = std::max(hi, pos(t, a)); }
+      const int edge = (a == 0 ? g.tx : a == 1 ? g.ty : g.tz) * (hi - lo + 1);
+      if (hi >= 0 && edge > longest) { longest = edge; axis = a; }
+    }
+    std::stable_sort(p.tiles.begin(), p.tiles.end(), [&](int a, int b) { return pos(a, axis) < pos(b, axis); });
+    const int mid = (p.lo + p.hi) / 2;
+    size_t share = 0;
+    for (int x = p.lo; x < mid; ++x) share += slots[x].size();
+    todo.push_back({std::vector<int>(p.tiles.begin(), p.tiles.begin() + (long)share), p.lo, mid});
+    todo.push_back({std::vector<int>(p.tiles.begin() + (long)share, p.tiles.end()), mid, p.hi});
+  }
+}
+
+// The instances of a level that the block-resident sweep runs, as groups split
+// into launches of at most kBlkCapacity tiles.  One voxel per thread
+// where all tiles then fit the chip at once (the shortest iteration), two
+// otherwise.  `tables`: the work-groups' table too, which sizing does not need.
+// Returns the exchange buffer's entries.
+static size_t choose_blocks(LevelPlan& L, bool tables) {
+  const int n = (int)L.host.size();
+  L.blk_groups.clear();
+  L.blk_launches.clear();
+  L.rest.clear();
+  std::map<std::array<int, 3>, BlockGroup> shapes;
+  for (int v = 1; v <= 2; ++v) {
+    shapes.clear();
+    bool all = true;
+    int64_t tiles = 0;
+    for (auto& d : L.host) {
+      const std::array<int, 3> key{d.NZ, d.NY, d.NX};
+      auto it = shapes.find(key);
+      if (it == shapes.end()) {
+        BlockGroup g{};
+        if (!block_shape_v(v, d, v == 1, &g)) g.tx = 0;
+        it = shapes.emplace(key, g).first;
+      }
+      all = all && it->second.tx > 0;
+      tiles += it->second.tx ? block_tiles(it->second) : 0;
+    }
+    L.blk_v = v;
+    if (all && tiles <= kBlkCapacity) break;
+  }
+  size_t box = 0, most = 0;
+  for (int k = 0; k < n; ++k) {
+    const LevelDesc& d = L.host[k];
+    BlockGroup g = shapes[{d.NZ, d.NY, d.NX}];
+    if (!g.tx) {
+      L.rest.push_back(k);
+      continue;
+    }
+    const int t = block_tiles(g);
+    if (L.blk_launches.empty() || L.blk_launches.back().tiles + t > kBlkCapacity) {
+      L.blk_launches.push_back({(int)L.blk_groups.size(), 0, 0});
+      box = 0;
+    }
+    LevelPlan::BlockLaunch& b = L.blk_launches.back();
+    g.inst = k;
+    g.first = b.tiles;
+    g.box = (unsigned)box;
+    box += (size_t)t * block_entries(g);
+    most = std::max(most, box);
+    b.tiles += t;
+    b.ngroups++;
+    L.blk_groups.push_back(g);
+  }
+  L.blk_tiles.clear();
+  if (!tables) return most;
+  std::map<std::array<int, 4>, std::vector<int>> dealt;  // by size and first XCD
+  for (const LevelPlan::BlockLaunch& b : L.blk_launches)
+    for (int k = 0; k < b.ngroups; ++k) {
+      const BlockGroup& g = L.blk_groups[b.first + k];
+      const LevelDesc& d = L.host[g.inst];
+      std::vector<int>& at = dealt[{d.NZ, d.NY, d.NX, g.first % kXcds}];
+      std::vector<int> wg(block_tiles(g));
+      if (at.empty()) deal_tiles(g, at);
+      for (size_t w = 0; w < at.size(); ++w) wg[at[w]] = (int)w;
+      for (int t : at) {
+        BlockTile c{};
+        c.group = (short)k;
+        c.bx = (short)(t % g.ntx);
+        c.by = (short)((t / g.ntx) % g.nty);
+        c.bz = (short)(t / (g.ntx * g.nty));
+        const int hop[3] = {1, g.ntx, g.ntx * g.nty}, pos[3] = {c.bx, c.by, c.bz}, size[3] = {g.ntx, g.nty, g.ntz};
+        for (int a = 0; a < 3; ++a) {
+          c.nb[2 * a] = (short)(pos[a] > 0 ? g.first + wg[t - hop[a]] : -1);
+          c.nb[2 * a + 1] = (short)(pos[a] + 1 < size[a] ? g.first + wg[t + hop[a]] : -1);
+        }
+        L.blk_tiles.push_back(c);
+      }
+    }
+  return most;
+}
+
 }  // namespace svs
 
 using namespace svs;
@@ -1201,6 +1434,13 @@ using namespace svs;
 // The extended model (Huber-TV, over-relaxation; no reference counterpart):
 // its sweeps keep the over-relaxed point z in fields of its own.
 static bool extended_model(const svs_tvl1_params& P) { return P.huber_eps > 0.0 || P.relax_theta != 0.0; }
+
+// Levels may run the block-resident sweep: the reference's model, no pinned
+// marching shape, something to iterate.
+static bool may_block(const svs_tvl1_params& P) {
+  return !extended_model(P) && P.sweep_bx <= 0 && P.sweep_by <= 0 && P.sweep_cz <= 0 && P.max_outer_iterations > 0 &&
+         P.max_warps > 0 && P.max_outer_iterations <= (1 << 24);  // sequence numbers have 32 bits
+}
 
 // Workspace layout, computed identically by the sizing and the plan builder.
 static int plan_layout(svs_plan* pl, char* base, size_t* total_out) {
@@ -1250,6 +1490,8 @@ static int plan_layout(svs_plan* pl, char* base, size_t* total_out) {
     }
   }
   // Device tables.
+  size_t box_entries = 0, max_groups = 0;
+  pl->blk_need = 0;
   for (int s = 0; s < S; ++s) {
     LevelPlan& L = pl->levels[s];
     choose_sweep_shape(P, L, pl->ninst);
@@ -1293,6 +1535,29 @@ static int plan_layout(svs_plan* pl, char* base, size_t* total_out) {
         if (it != g_tuned_resident.end() && !it->second) L.resident = 0;
       }
     }
+    L.blk_capable = L.blk_on = false;
+    if (may_block(P) && !L.res_capable) {
+      box_entries = std::max(box_entries, choose_blocks(L, base != nullptr));
+      if (!L.blk_groups.empty()) {
+        L.blk_capable = L.blk_on = true;
+        {  // unless the autotuner measured the marching sweep faster
+          std::lock_guard<std::mutex> lk(g_tune_mu);
+          auto it = g_tuned_blocks.find(tune_key(P, L));
+          if (it != g_tuned_blocks.end()) L.blk_on = it->second;
+        }
+        L.blk_dev = (BlockGroup*)take(sizeof(BlockGroup) * L.blk_groups.size());
+        size_t tiles = 0;
+        for (auto& b : L.blk_launches) tiles += b.tiles;
+        L.blk_tiles_dev = (BlockTile*)take(sizeof(BlockTile) * tiles);
+        if (!L.rest.empty()) {
+          L.rest_dev = (int*)take(sizeof(int) * L.rest.size());
+          L.rest_tiles = (SweepTile*)take(sizeof(SweepTile) * cap);
+        }
+        for (auto& b : L.blk_launches)  // whole rounds of the 8 XCDs' 4 shader engines
+          pl->blk_need = std::max(pl->blk_need, (b.tiles + 31) / 32 * 32);
+        max_groups = std::max(max_groups, L.blk_groups.size());
+      }
+    }
     L.px_blocks = L.py_blocks = 0;
     if (s + 1 < S)
       for (int k = 0; k < pl->ninst; ++k) {
@@ -1302,6 +1567,12 @@ static int plan_layout(svs_plan* pl, char* base, size_t* total_out) {
   }
   if (P.use_blur) pl->blur_dev = (float*)take(sizeof(float) * pl->blur_w.size());
   pl->sched_dev = (float*)take(sizeof(float) * 4 * (size_t)std::max(1, P.max_outer_iterations));
+  if (max_groups) {
+    pl->blk_ctl = (BlockCtl*)take(sizeof(BlockCtl));
+    pl->blk_done = (BlockDone*)take(sizeof(BlockDone) * max_groups);
+    pl->blk_box_bytes = sizeof(u64) * box_entries;
+    pl->blk_box = (u64*)take(pl->blk_box_bytes);
+  }
   *total_out = align_up(off, 256);
   return 0;
 }
@@ -1419,9 +1690,12 @@ static void drop_graph(svs_plan* pl) {
   if (pl->graph) { (void)hipGraphDestroy(pl->graph); pl->graph = nullptr; }
 }
 
+static void forget_run(svs_plan* pl);
+
 // Releases the plan's resources once its last work has completed.
 static void free_plan(svs_plan* pl) {
   if (pl->last_work) (void)hipEventSynchronize(pl->last_work);
+  forget_run(pl);  // only now: until here other plans' runs still wait for this one's
   for (int i = 0; i < svs_plan::kStagingSlots; ++i)
     if (pl->staged[i]) {
       (void)hipEventSynchronize(pl->staged[i]);
@@ -1438,7 +1712,10 @@ static void free_plan(svs_plan* pl) {
 
 static int create_sync_objects(svs_plan* pl) {
   pl->table_bytes = sizeof(LevelDesc) * (size_t)pl->ninst * pl->S;
-  SVS_HIP(hipHostMalloc((void**)&pl->staging, pl->table_bytes * svs_plan::kStagingSlots, hipHostMallocDefault));
+  const size_t staged = pl->table_bytes * svs_plan::kStagingSlots;
+  SVS_HIP(hipHostMalloc((void**)&pl->staging, staged + sizeof(unsigned), hipHostMallocDefault));
+  pl->blk_redone = (unsigned*)((char*)pl->staging + staged);
+  *pl->blk_redone = 0;
   SVS_HIP(hipEventCreateWithFlags(&pl->last_work, hipEventDisableTiming));
   for (int i = 0; i < svs_plan::kStagingSlots; ++i)
     SVS_HIP(hipEventCreateWithFlags(&pl->staged[i], hipEventDisableTiming));
@@ -1498,30 +1775,30 @@ static int upload_tiles(svs_plan* pl, int s, hipStream_t st) {
     LevelPlan& L = pl->levels[s];
     L.ntiles = count_tiles(L, L.bx, L.by, L.cz);
     SVS_REQUIRE(L.ntiles <= L.tile_capacity, "tile table overflow (%d > %d)", L.ntiles, L.tile_capacity);
-    std::vector<SweepTile> natural;
-    natural.reserve(L.ntiles);
     L.threads = 0;
     L.lds = 0;
-    for (int k = 0; k < pl->ninst; ++k) {
-      const LevelDesc& d = L.host[k];
-      int tbx, tby;
-      inst_tile(d, L.bx, L.by, tbx, tby);
-      L.threads = std::max(L.threads, tbx * tby);
-      L.lds = std::max(L.lds, sweep_lds_bytes(tbx, tby));
-      const int tx = tbx - 2, ty = tby - 2;
-      for (int z0 = 0; z0 < d.NZ; z0 += L.cz)
-        for (int y0 = 0; y0 < d.NY; y0 += ty)
-          for (int x0 = 0; x0 < d.NX; x0 += tx) {
-            const int z1 = std::min(d.NZ, z0 + L.cz);
-            natural.push_back(SweepTile{k, x0 | (y0 << 16), z0 | (z1 << 16), tbx | (tby << 16)});
-          }
-    }
-    // Work-group b runs on XCD b % 8.  Deal contiguous runs of the natural
-    // order (neighbouring tiles of one volume) to one XCD each, so the halo
-    // rows a tile re-reads from its neighbours sit in the same L2.
-    std::vector<SweepTile> tiles;
-    tiles.reserve(natural.size());
-    {
+    // The tiles of the listed instances in launch order.
+    auto tiles_of = [&](const std::vector<int>& insts) {
+      std::vector<SweepTile> natural;
+      for (int k : insts) {
+        const LevelDesc& d = L.host[k];
+        int tbx, tby;
+        inst_tile(d, L.bx, L.by, tbx, tby);
+        L.threads = std::max(L.threads, tbx * tby);
+        L.lds = std::max(L.lds, sweep_lds_bytes(tbx, tby));
+        const int tx = tbx - 2, ty = tby - 2;
+        for (int z0 = 0; z0 < d.NZ; z0 += L.cz)
+          for (int y0 = 0; y0 < d.NY; y0 += ty)
+            for (int x0 = 0; x0 < d.NX; x0 += tx) {
+              const int z1 = std::min(d.NZ, z0 + L.cz);
+              natural.push_back(SweepTile{k, x0 | (y0 << 16), z0 | (z1 << 16), tbx | (tby << 16)});
+            }
+      }
+      // Work-group b runs on XCD b % 8.  Deal contiguous runs of the natural
+      // order (neighbouring tiles of one volume) to one XCD each, so the halo
+      // rows a tile re-reads from its neighbours sit in the same L2.
+      std::vector<SweepTile> tiles;
+      tiles.reserve(natural.size());
       const int nx = kXcds, n = (int)natural.size();
       std::vector<int> start(nx + 1);
       for (int g = 0; g <= nx; ++g) start[g] = (int)((int64_t)n * g / nx);
@@ -1529,6 +1806,16 @@ static int upload_tiles(svs_plan* pl, int s, hipStream_t st) {
       for (int slot = 0; slot < maxlen; ++slot)
         for (int g = 0; g < nx; ++g)
           if (start[g] + slot < start[g + 1]) tiles.push_back(natural[start[g] + slot]);
+      return tiles;
+    };
+    std::vector<int> every(pl->ninst);
+    for (int k = 0; k < pl->ninst; ++k) every[k] = k;
+    const std::vector<SweepTile> tiles = tiles_of(every);
+    std::vector<SweepTile> rest;
+    if (L.rest_tiles) {
+      rest = tiles_of(L.rest);
+      L.nrest_tiles = (int)rest.size();
+      SVS_HIP(hipMemcpyAsync(L.rest_tiles, rest.data(), sizeof(SweepTile) * rest.size(), hipMemcpyHostToDevice, st));
     }
     SVS_HIP(hipMemcpyAsync(L.tiles, tiles.data(), sizeof(SweepTile) * tiles.size(), hipMemcpyHostToDevice, st));
     // Each instance's tiles in launch order, for the statistics reduction.
@@ -1551,16 +1838,19 @@ struct SweepScalars {
   float sg, ta, fac, wtv, hub, eps, theta;
   int zfirst;
   bool ext;
+  bool rest;  // the instances the block-resident sweep leaves
 };
 
 template <int BC, bool ANISO, bool STATS, bool EXT>
 static void launch_sweep_s(const LevelPlan& L, int parity, const SweepScalars& a, float4* part, hipStream_t st) {
+  const SweepTile* tiles = a.rest ? L.rest_tiles : L.tiles;
+  const int ntiles = a.rest ? L.nrest_tiles : L.ntiles;
   if (L.unit_h)
-    hipLaunchKernelGGL((k_sweep<BC, ANISO, true, STATS, EXT>), dim3(L.ntiles), dim3(L.threads), L.lds, st, L.dev,
-                       L.tiles, parity, a.sg, a.ta, a.fac, a.wtv, a.hub, a.eps, a.theta, a.zfirst, part);
+    hipLaunchKernelGGL((k_sweep<BC, ANISO, true, STATS, EXT>), dim3(ntiles), dim3(L.threads), L.lds, st, L.dev,
+                       tiles, parity, a.sg, a.ta, a.fac, a.wtv, a.hub, a.eps, a.theta, a.zfirst, part);
   else
-    hipLaunchKernelGGL((k_sweep<BC, ANISO, false, STATS, EXT>), dim3(L.ntiles), dim3(L.threads), L.lds, st,
-                       L.dev, L.tiles, parity, a.sg, a.ta, a.fac, a.wtv, a.hub, a.eps, a.theta, a.zfirst, part);
+    hipLaunchKernelGGL((k_sweep<BC, ANISO, false, STATS, EXT>), dim3(ntiles), dim3(L.threads), L.lds, st,
+                       L.dev, tiles, parity, a.sg, a.ta, a.fac, a.wtv, a.hub, a.eps, a.theta, a.zfirst, part);
 }
 
 template <int BC, bool ANISO>
@@ -1577,10 +1867,10 @@ static void launch_sweep_t(const LevelPlan& L, int parity, const SweepScalars& a
 // One sweep at schedule position n; part (null: no statistics) receives one
 // float4 of statistics sums per work-group.
 static void launch_sweep(const svs_plan* pl, const LevelPlan& L, int parity, int n, hipStream_t st,
-                         float4* part = nullptr) {
+                         float4* part = nullptr, bool rest = false) {
   const svs_tvl1_params& P = pl->P;
   const SweepScalars a{pl->sig[n], pl->tau[n], pl->factor[n], P.weight_tv, pl->hub[n], (float)P.huber_eps,
-                       (float)P.relax_theta, n == 0 ? 1 : 0, extended_model(P)};
+                       (float)P.relax_theta, n == 0 ? 1 : 0, extended_model(P), rest};
   const bool an = P.use_aniso != 0;
   switch (P.boundary * 2 + (an ? 1 : 0)) {
     case 0: launch_sweep_t<BD_NEAREST, false>(L, parity, a, part, st); break;
@@ -1629,6 +1919,134 @@ static void launch_resident(const svs_plan* pl, const LevelPlan& L, int parity, 
     case 4: launch_resident_t<BD_REFLECT, false>(pl, L, parity, first, K, part, st); break;
     default: launch_resident_t<BD_REFLECT, true>(pl, L, parity, first, K, part, st); break;
   }
+}
+
+template <int BC, bool ANISO>
+static const void* block_kernel_t(bool unit_h, int v) {
+  if (v == 1)
+    return unit_h ? (const void*)k_sweep_block<BC, ANISO, true, 1> : (const void*)k_sweep_block<BC, ANISO, false, 1>;
+  return unit_h ? (const void*)k_sweep_block<BC, ANISO, true, 2> : (const void*)k_sweep_block<BC, ANISO, false, 2>;
+}
+
+// The block-resident sweep's kernel for a level, and its dynamic LDS.
+static const void* block_kernel(const svs_plan* pl, const LevelPlan& L) {
+  switch (pl->P.boundary * 2 + (pl->P.use_aniso ? 1 : 0)) {
+    case 0: return block_kernel_t<BD_NEAREST, false>(L.unit_h, L.blk_v);
+    case 1: return block_kernel_t<BD_NEAREST, true>(L.unit_h, L.blk_v);
+    case 2: return block_kernel_t<BD_MIRROR, false>(L.unit_h, L.blk_v);
+    case 3: return block_kernel_t<BD_MIRROR, true>(L.unit_h, L.blk_v);
+    case 4: return block_kernel_t<BD_REFLECT, false>(L.unit_h, L.blk_v);
+    default: return block_kernel_t<BD_REFLECT, true>(L.unit_h, L.blk_v);
+  }
+}
+static size_t block_lds(const LevelPlan& L) { return L.blk_v == 1 ? blk_lds_bytes<1>() : blk_lds_bytes<2>(); }
+
+// One warp's K iterations of the level's block-resident instances, from state
+// buffer `parity` into the other one.
+static int launch_blocks(const svs_plan* pl, const LevelPlan& L, int parity, hipStream_t st) {
+  const void* kernel = block_kernel(pl, L);
+  const LevelDesc* descs = L.dev;
+  const float* sched = pl->sched_dev;
+  int K = pl->P.max_outer_iterations;
+  float wtv = pl->P.weight_tv;
+  u64* box = pl->blk_box;
+  BlockCtl* ctl = pl->blk_ctl;
+  BlockDone* done = pl->blk_done;
+  u64 ticks = pl->blk_wait_ticks;
+  unsigned* redone = pl->blk_redone;
+  const BlockTile* tiles = L.blk_tiles_dev;
+  for (const LevelPlan::BlockLaunch& b : L.blk_launches) {
+    const BlockGroup* groups = L.blk_dev + b.first;
+    int ngroups = b.ngroups;
+    void* args[] = {&descs, &groups, &tiles, &ngroups, &sched, &K, &parity, &wtv, &box, &ctl, &done, &ticks,
+                    &redone};
+    SVS_HIP(hipLaunchKernel(kernel, dim3(b.tiles), dim3(kBlkThreads), args, block_lds(L), st));
+    tiles += b.tiles;
+  }
+  return 0;
+}
+
+// Switches the block-resident sweep off where the device does not hold
+// kBlkCapacity of its work-groups at once, and clears its counters.
+static int prepare_blocks(svs_plan* pl, hipStream_t st) {
+  SVS_HIP(hipGetDevice(&pl->device));
+  if (!pl->blk_need) return 0;
+  int cus = 0;
+  SVS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, pl->device));
+  bool any = false;
+  size_t groups = 1;
+  for (LevelPlan& L : pl->levels) {
+    if (!L.blk_capable) continue;
+    const void* kernel = block_kernel(pl, L);
+    SVS_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)block_lds(L)));
+    int per_cu = 0;
+    SVS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlkThreads, block_lds(L)));
+    if (per_cu * cus < kBlkCapacity) {
+      L.blk_capable = L.blk_on = false;
+      continue;
+    }
+    any = true;
+    groups = std::max(groups, L.blk_groups.size());
+    SVS_HIP(hipMemcpyAsync(L.blk_dev, L.blk_groups.data(), sizeof(BlockGroup) * L.blk_groups.size(),
+                           hipMemcpyHostToDevice, st));
+    SVS_HIP(hipMemcpyAsync(L.blk_tiles_dev, L.blk_tiles.data(), sizeof(BlockTile) * L.blk_tiles.size(),
+                           hipMemcpyHostToDevice, st));
+    if (!L.rest.empty())
+      SVS_HIP(hipMemcpyAsync(L.rest_dev, L.rest.data(), sizeof(int) * L.rest.size(), hipMemcpyHostToDevice, st));
+  }
+  if (!any) {
+    pl->blk_need = 0;
+    return 0;
+  }
+  if (int rc = launch_fill((float*)pl->blk_ctl, sizeof(BlockCtl) / 4, 0.0f, st)) return rc;
+  if (int rc = launch_fill((float*)pl->blk_done, (int64_t)(sizeof(BlockDone) / 4 * groups), 0.0f, st)) return rc;
+  if (int rc = launch_fill((float*)pl->blk_box, (int64_t)(pl->blk_box_bytes / 4), 0.0f, st)) return rc;
+  SVS_HIP(hipStreamSynchronize(st));
+  return 0;
+}
+
+// Work-groups of one group wait for each other, so launches of different
+// streams may run at once only if all their work-groups fit the device
+// together.  Runs whose plan uses the block-resident sweep are kept in order of
+// enqueueing per device; a new one waits for every earlier run outside the
+// longest recent stretch that fits beside it, whatever streams and threads
+// they came from.  (Another process on the device is not seen here; then the
+// waits' time limit decides.)
+static std::mutex g_runs_mu;
+static std::map<int, std::vector<svs_plan*>> g_runs;  // oldest first, each plan once
+
+static int wait_turn(svs_plan* pl, hipStream_t st) {
+  std::vector<svs_plan*>& runs = g_runs[pl->device];
+  int room = kBlkCapacity - pl->blk_need;
+  bool fits = true;
+  for (size_t i = runs.size(); i-- > 0;) {
+    svs_plan* o = runs[i];
+    if (o == pl) continue;
+    fits = fits && o->blk_need <= room;
+    if (fits) {
+      room -= o->blk_need;
+      continue;
+    }
+    const hipError_t e = hipEventQuery(o->last_work);
+    if (e == hipSuccess) {
+      runs.erase(runs.begin() + (long)i);
+      continue;
+    }
+    (void)hipGetLastError();  // hipErrorNotReady
+    SVS_HIP(hipStreamWaitEvent(st, o->last_work, 0));
+  }
+  return 0;
+}
+
+static void note_run(svs_plan* pl, bool keep) {
+  std::vector<svs_plan*>& runs = g_runs[pl->device];
+  runs.erase(std::remove(runs.begin(), runs.end(), pl), runs.end());
+  if (keep) runs.push_back(pl);
+}
+
+static void forget_run(svs_plan* pl) {
+  std::lock_guard<std::mutex> lk(g_runs_mu);
+  note_run(pl, false);
 }
 
 template <int BC, bool ANISO>
@@ -1712,7 +2130,7 @@ static int ensure_stats_part(svs_plan* pl) {
 }
 
 // Enqueues the complete solve of every instance on one stream.
-static int enqueue_solve(svs_plan* pl, hipStream_t st) {
+static int enqueue_solve(svs_plan* pl, hipStream_t st, bool blocks = true) {
   const svs_tvl1_params& P = pl->P;
   const int S = pl->S, n = pl->ninst;
   const int ip = P.interpolation, bc = P.boundary;
@@ -1754,6 +2172,22 @@ static int enqueue_solve(svs_plan* pl, hipStream_t st) {
           SVS_LAUNCHED();
         }
         parity ^= K & 1;
+        continue;
+      }
+      if (L.blk_on && blocks && !sout) {
+        if (int rc = launch_blocks(pl, L, parity, st)) return rc;
+        if (!L.rest.empty()) {
+          const int nr = (int)L.rest.size();
+          for (int it = 0; it < K; ++it) {
+            launch_sweep(pl, L, parity ^ (it & 1), it, st, nullptr, true);
+            SVS_LAUNCHED();
+          }
+          if (!(K & 1)) {
+            k_swap_state<<<(nr + 63) / 64, 64, 0, st>>>(L.dev, L.rest_dev, nr);
+            SVS_LAUNCHED();
+          }
+        }
+        parity ^= 1;
         continue;
       }
       for (int it = 0; it < K; ++it) {
@@ -1838,6 +2272,7 @@ int svs_tvl1_plan_create(const svs_tvl1_params* P, int ninst, const int* dims, v
   if (int rc = allow_large_lds(pl)) { delete pl; return rc; }
   if (int rc = create_sync_objects(pl)) { free_plan(pl); return rc; }
   hipStream_t st = (hipStream_t)stream;
+  if (int rc = prepare_blocks(pl, st)) { free_plan(pl); return rc; }
   if (int rc = upload_static(pl, st)) { free_plan(pl); return rc; }
   if (int rc = mark_last_work(pl, st)) { free_plan(pl); return rc; }
   *out = pl;
@@ -1873,9 +2308,32 @@ int svs_tvl1_plan_run(svs_plan* pl, int use_graph, void* stream) {
   if (int rc = after_last_work(pl, st)) return rc;
   if (pl->tables_dirty)
     if (int rc = upload_tables(pl, st)) return rc;
-  if (!use_graph) {
-    if (int rc = enqueue_solve(pl, st)) return rc;
+  // A run that the caller records into a graph of its own takes the marching
+  // sweep: its replays would not be kept apart from other plans' runs.
+  hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
+  if (pl->blk_need && !use_graph && hipStreamIsCapturing(st, &recording) != hipSuccess) (void)hipGetLastError();
+  if (recording == hipStreamCaptureStatusActive) {
+    if (int rc = enqueue_solve(pl, st, false)) return rc;
     return mark_last_work(pl, st);
+  }
+  if (pl->blk_need && *(volatile unsigned*)pl->blk_redone) {  // an earlier run's waits were given up
+    for (LevelPlan& L : pl->levels) L.blk_on = false;
+    drop_graph(pl);
+    *pl->blk_redone = 0;
+  }
+  std::unique_lock<std::mutex> turn(g_runs_mu, std::defer_lock);
+  if (pl->blk_need) {  // held until the run and its event are enqueued
+    turn.lock();
+    if (int rc = wait_turn(pl, st)) return rc;
+  }
+  auto ran = [&]() {
+    if (pl->blk_need) note_run(pl, true);
+    return mark_last_work(pl, st);
+  };
+  if (!use_graph) {
+    const int rc = enqueue_solve(pl, st);
+    const int rm = ran();
+    return rc ? rc : rm;
   }
   if (!pl->exec) {
     if (!pl->capture_stream) SVS_HIP(hipStreamCreateWithFlags(&pl->capture_stream, hipStreamNonBlocking));
@@ -1889,7 +2347,7 @@ int svs_tvl1_plan_run(svs_plan* pl, int use_graph, void* stream) {
     SVS_HIP(hipGraphInstantiate(&pl->exec, pl->graph, nullptr, nullptr, 0));
   }
   SVS_HIP(hipGraphLaunch(pl->exec, st));
-  return mark_last_work(pl, st);
+  return ran();
 }
 
 int svs_tvl1_plan_destroy(svs_plan* pl) {
@@ -2039,9 +2497,30 @@ int svs_tvl1_plan_autotune(svs_plan* pl, int reps, void* stream, int* report /* 
       resident_wins = ms_res / K < best_ms / reps;
       L.resident = resident_wins ? L.res_capable : 0;
     }
+    // The same choice where every instance fits the block-resident sweep.
+    bool blocks_win = false;
+    const bool choose = L.blk_capable && L.rest.empty();
+    if (choose) {
+      std::lock_guard<std::mutex> turn(g_runs_mu);
+      if ((rc = wait_turn(pl, st))) break;
+      float ms_blk = 0.0f;
+      auto time_blocks = [&]() -> int {
+        if (int r = launch_blocks(pl, L, 0, st)) return r;
+        SVS_HIP(hipEventRecord(e0, st));
+        if (int r = launch_blocks(pl, L, 0, st)) return r;
+        SVS_HIP(hipEventRecord(e1, st));
+        SVS_HIP(hipEventSynchronize(e1));
+        SVS_HIP(hipEventElapsedTime(&ms_blk, e0, e1));
+        return 0;
+      };
+      if ((rc = time_blocks())) break;
+      blocks_win = ms_blk / (float)pl->P.max_outer_iterations < best_ms / (float)reps;
+      L.blk_on = blocks_win;
+    }
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[tune_key(pl->P, L)] = best;
     if (L.res_capable) g_tuned_resident[tune_key(pl->P, L)] = resident_wins;
+    if (choose) g_tuned_blocks[tune_key(pl->P, L)] = blocks_win;
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -2060,9 +2539,34 @@ int svs_tvl1_plan_set_shape(svs_plan* pl, int level, int bx, int by, int cz, voi
   hipStream_t st = (hipStream_t)stream;
   if (int rc = after_last_work(pl, st)) return rc;
   L.bx = bx; L.by = by; L.cz = cz;
+  L.blk_on = false;
   if (int rc = upload_tiles(pl, level, st)) return rc;
   drop_graph(pl);
   return mark_last_work(pl, st);
+}
+
+int svs_tvl1_plan_blocks(const svs_plan* pl, int level, int* out /* 5 ints */) {
+  SVS_REQUIRE(pl && level >= 0 && level < pl->S && out, "bad plan/level");
+  const LevelPlan& L = pl->levels[level];
+  out[0] = L.blk_on ? (int)L.blk_groups.size() : 0;
+  out[1] = L.blk_v;
+  out[2] = 0;
+  for (const BlockGroup& g : L.blk_groups) out[2] = std::max(out[2], block_tiles(g));
+  out[3] = (int)L.blk_launches.size();
+  out[4] = 0;
+  if (pl->blk_need) {
+    SVS_HIP(hipEventSynchronize(pl->last_work));
+    SVS_HIP(hipMemcpy(&out[4], &pl->blk_ctl->redone, sizeof(unsigned), hipMemcpyDeviceToHost));
+  }
+  return 0;
+}
+
+int svs_tvl1_plan_set_wait_limit(svs_plan* pl, int microseconds, void* stream) {
+  SVS_REQUIRE(pl && microseconds >= 0, "bad plan or wait limit");
+  if (int rc = after_last_work(pl, (hipStream_t)stream)) return rc;
+  pl->blk_wait_ticks = (unsigned long long)microseconds * 100ull;  // 100 MHz clock
+  drop_graph(pl);
+  return mark_last_work(pl, (hipStream_t)stream);
 }
 
 int svs_tvl1_plan_set_stats(svs_plan* pl, float* out, void* stream) {
@@ -2097,6 +2601,7 @@ int svs_tvl1_plan_set_resident(svs_plan* pl, int level, int mode, void* stream) 
   hipStream_t st = (hipStream_t)stream;
   if (int rc = after_last_work(pl, st)) return rc;
   L.resident = mode == 0 ? 0 : L.res_capable;
+  L.blk_on = mode != 0 && L.blk_capable;
   drop_graph(pl);
   return mark_last_work(pl, st);
 }

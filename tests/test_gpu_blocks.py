@@ -1,0 +1,113 @@
+"""The block-resident sweep (an instance's state held on chip by several
+work-groups) gives the marching sweep's bits; the marching sweep equals the
+FP32 oracle's (test_gpu_solver.py, whose volumes of more than 2048 voxels also
+run block-resident)."""
+import ctypes
+
+import pytest
+import torch
+
+from singleventriclesegmentation_amd import _lib
+from singleventriclesegmentation_amd.solver import Plan, SolverConfig
+
+pytestmark = pytest.mark.gpu
+
+
+def _blocks(plan):
+    out = (ctypes.c_int * 5)()
+    _lib.check(_lib.lib().svs_tvl1_plan_blocks(plan._h, 0, out))
+    return list(out)  # instances, voxels per thread, work-groups of the largest, launches, redone
+
+
+def _plan(dev, cfg, shapes, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    plan, outs = Plan(cfg, shapes), []
+    for k, s in enumerate(shapes):
+        z, y, x = torch.meshgrid(*(torch.linspace(0, 3, n) for n in s), indexing="ij")
+        f = [torch.sin(2 * x + k + d) * torch.cos(3 * y - d) + z + 0.05 * torch.rand(s, generator=g) for d in (0.0, 0.3)]
+        u, p = torch.empty(s + (3,), device=dev), torch.empty(s + (3, 3), device=dev)
+        plan.bind(k, f[0].to(dev), f[1].to(dev), u_out=u, p_out=p)
+        outs += [u, p]
+    return plan, outs
+
+
+def _config(K, boundary, aniso, length=None, warps=2):
+    return SolverConfig(num_scales=1, max_warps=warps, max_outer_iterations=K, boundary=boundary, use_aniso=aniso,
+                        length_fixed=length is not None, length=length or (1.0, 1.0, 1.0))
+
+
+# Sizes, K, boundary (0 nearest, 1 mirror, 2 reflect), anisotropy, mesh lengths;
+# expected: instances block-resident, voxels per thread, launches per warp.
+CASES = [
+    ([(13, 15, 14)], 5, 1, True, None, (1, 1, 1)),                 # just above the resident sweep's range
+    ([(4, 70, 11)], 4, 0, True, None, (1, 1, 1)),                  # the smallest extent along z
+    ([(47, 4, 53)], 5, 2, False, None, (1, 1, 1)),                 # and along another
+    ([(29, 31, 30)], 1, 2, True, None, (1, 1, 1)),                 # a single iteration, ragged last tiles
+    ([(33, 34, 35)], 6, 1, False, (17.0, 40.0, 25.0), (1, 1, 1)),  # h != 1, nearly all work-groups
+    ([(60, 71, 70)], 5, 1, True, None, (1, 2, 1)),                 # two voxels per thread, ragged
+    ([(80, 80, 80)], 4, 0, True, None, (1, 2, 1)),                 # every work-group of the device
+    ([(71, 67, 75)], 4, 2, False, (50.0, 67.0, 90.0), (1, 2, 1)),
+    ([(40, 40, 40)] * 9 + [(20, 24, 22), (61, 47, 75)], 5, 1, True, None, (11, 2, 2)),    # groups over launches
+    ([(20, 24, 22), (84, 90, 70), (4, 4, 2000)], 4, 1, True, None, (2, 2, 1)),  # some instances do not fit: even K
+    ([(20, 24, 22), (84, 90, 70)], 5, 0, False, None, (1, 2, 1)),               # and odd
+]
+
+
+@pytest.mark.parametrize("shapes,K,boundary,aniso,length,expected", CASES)
+def test_blocks_equal_marching(dev, shapes, K, boundary, aniso, length, expected):
+    cfg = _config(K, boundary, aniso, length)
+    plan, got = _plan(dev, cfg, shapes)
+    b = _blocks(plan)
+    assert (b[0], b[1], b[3]) == expected
+    runs = []
+    for _ in range(2):  # the second run reuses exchange buffer and counters
+        plan.run()
+        torch.cuda.synchronize()
+        runs.append([t.clone() for t in got])
+    assert _blocks(plan)[4] == 0
+    plan.set_resident(0, 0)
+    plan.run()
+    torch.cuda.synchronize()
+    for first, second, marching in zip(runs[0], runs[1], got):
+        assert torch.equal(first, marching) and torch.equal(second, marching)
+    plan.close()
+
+
+@pytest.mark.parametrize("shape,K", [((20, 24, 22), 5), ((60, 71, 70), 4)])
+def test_blocks_redone_by_one_work_group(dev, shape, K):
+    """With no patience for a neighbour an instance is redone by one
+    work-group: the same bits, and the next run marches."""
+    plan, got = _plan(dev, _config(K, 1, True), [shape])
+    plan.run()
+    torch.cuda.synchronize()
+    want = [t.clone() for t in got]
+    _lib.check(_lib.lib().svs_tvl1_plan_set_wait_limit(plan._h, 0, _lib.stream_ptr()))
+    for on in (1, 0):
+        plan.run()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        assert _blocks(plan)[4] > 0
+    assert _blocks(plan)[0] == 0
+    plan.close()
+
+
+def test_blocks_on_several_streams(dev):
+    """Plans that fill the device, or half of it, run from three streams at
+    once without disturbing each other."""
+    cfg = _config(20, 1, True, warps=3)
+    work = [_plan(dev, cfg, [s], seed=i) for i, s in enumerate([(80, 80, 80), (40, 40, 40), (64, 50, 40)])]
+    want = []
+    for plan, got in work:
+        plan.run()
+        torch.cuda.synchronize()
+        want.append([t.clone() for t in got])
+    streams = [torch.cuda.Stream(device=dev) for _ in work]
+    for r in range(6):
+        for (plan, got), st in zip(work, streams):
+            with torch.cuda.stream(st):
+                plan.run(use_graph=r % 2 == 0)
+    torch.cuda.synchronize()
+    for (plan, got), w in zip(work, want):
+        assert all(torch.equal(a, b) for a, b in zip(got, w))
+        assert _blocks(plan)[0] == 1 and _blocks(plan)[4] == 0
+        plan.close()
