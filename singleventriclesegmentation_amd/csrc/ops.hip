@@ -259,15 +259,10 @@ __device__ void warp_backward_cubic(const float* __restrict__ u, const Acc& acc,
     float gy[4];
     const float gwy = cr_local_backward(by[0], by[1], by[2], by[3], ly, gzd, gy);
     gphi[1] += gwy / hY;
-#pragma unroll 1
+#pragma unroll 2
     for (int dy = 0; dy < 4; ++dy) {
-      int y = ys[0];
-      float gyd = gy[0];
-#pragma unroll
-      for (int k = 1; k < 4; ++k) {
-        y = dy == k ? ys[k] : y;
-        gyd = dy == k ? gy[k] : gyd;
-      }
+      const int y = ys[dy];
+      const float gyd = gy[dy];
       float gx[4];
       const float gwx = cr_local_backward(U(z, y, xs[0]), U(z, y, xs[1]), U(z, y, xs[2]), U(z, y, xs[3]), lx,
                                           gyd, gx);
@@ -311,20 +306,23 @@ __device__ void warp_backward_linear(const float* __restrict__ u, const Acc& acc
 // flow gradient sums the per-channel adjoints in channel order.  grad_u must
 // be zero on entry (the launcher clears it).
 //
-// A work-group owns a kAdjTX x kAdjTY x kAdjTZ tile of voxels.  Per channel it
-// sums the scattered grad_u contributions in an LDS window that covers the
-// tile, a displacement margin of kAdjM voxels and the 2-voxel cubic footprint,
-// then adds each non-zero window cell to grad_u with one global atomic.  Taps
-// outside the window (larger displacements, far boundary reflections) go to
-// grad_u directly.  The reference also accumulates with float atomics, so
-// grad_u's low bits depend on the order in either case; grad_phi does not.
-// A 16 x 16 x 1 tile (256 threads, 163 VGPRs, no spills, 29 KiB window) with a
-// 2-voxel margin measured fastest on 4 x 4 x 80^3 (2.9 ms; 32 x 8 x 4 with a
-// 3-voxel margin, 1024 threads capped at 128 VGPRs, spilled and took 4.0 ms).
-constexpr int kAdjTX = 16, kAdjTY = 16, kAdjTZ = 1, kAdjM = 2;
-constexpr int kAdjThreads = kAdjTX * kAdjTY * kAdjTZ;
-constexpr int kAdjWX = kAdjTX + 2 * (kAdjM + 2), kAdjWY = kAdjTY + 2 * (kAdjM + 2), kAdjWZ = kAdjTZ + 2 * (kAdjM + 2);
-constexpr int kAdjWin = kAdjWX * kAdjWY * kAdjWZ;
+// A work-group owns a kAdjTX x kAdjTY x TZ tile of voxels, two threads each
+// (x, y) column of it.  Per channel it sums the scattered grad_u contributions
+// in an LDS window that covers the tile, a displacement margin of kAdjM voxels
+// and the 2-voxel cubic footprint, then adds each non-zero window cell to
+// grad_u with one global atomic.  Taps outside the window (larger
+// displacements, far boundary reflections) go to grad_u directly.  The
+// reference also accumulates with float atomics, so grad_u's low bits depend on
+// the order in either case; grad_phi does not.
+// The 64 LDS adds per voxel bound it.  The window holds doubles because a
+// float LDS add is served lane by lane on gfx950 (about 190 clocks per
+// wavefront, 50 for 16 lanes) and a double one is not (40).  4 x 4 x 80^3:
+// 2820 us with floats, 670 with doubles and one thread per column, 643 with two
+// (16 waves per CU against 8 to 12).
+constexpr int kAdjTX = 16, kAdjTY = 16, kAdjM = 2;
+constexpr int kAdjG = 2;  // threads of a column
+constexpr int kAdjThreads = kAdjTX * kAdjTY * kAdjG;
+constexpr int kAdjWX = kAdjTX + 2 * (kAdjM + 2), kAdjWY = kAdjTY + 2 * (kAdjM + 2);
 
 struct GlobalAcc {
   float* grad;
@@ -334,28 +332,33 @@ struct GlobalAcc {
   }
 };
 
+typedef __attribute__((address_space(3))) double* LdsDouble;
+
+template <int WZ>
 struct WindowAcc {
-  float* win;       // LDS, kAdjWZ x kAdjWY x kAdjWX
+  LdsDouble win;    // WZ x kAdjWY x kAdjWX
   int z0, y0, x0;   // volume index of window cell (0, 0, 0)
   GlobalAcc outside;
   __device__ void operator()(int z, int y, int x, float v) const {
     const int lz = z - z0, ly = y - y0, lx = x - x0;
-    if ((unsigned)lz < (unsigned)kAdjWZ && (unsigned)ly < (unsigned)kAdjWY && (unsigned)lx < (unsigned)kAdjWX)
-      atomicAdd(win + (lz * kAdjWY + ly) * kAdjWX + lx, v);
+    if ((unsigned)lz < (unsigned)WZ && (unsigned)ly < (unsigned)kAdjWY && (unsigned)lx < (unsigned)kAdjWX)
+      __builtin_amdgcn_ds_atomic_fadd_f64(win + (lz * kAdjWY + ly) * kAdjWX + lx, (double)v);
     else
       outside(z, y, x, v);
   }
 };
 
+template <int TZ>
 __global__ __launch_bounds__(kAdjThreads) void k_warp_backward(const float* __restrict__ u,
                                                                const float* __restrict__ phi,
                                                                const float* __restrict__ gout, int B, int C, int NZ,
                                                                int NY, int NX, float hZ, float hY, float hX, int ip,
                                                                int bc, float* __restrict__ grad_u,
                                                                float* __restrict__ grad_phi) {
-  __shared__ float win[kAdjWin];
+  constexpr int kWZ = TZ + 2 * (kAdjM + 2), kWin = kAdjWX * kAdjWY * kWZ;
+  __shared__ double win[kWin];
   const int tiles_x = (NX + kAdjTX - 1) / kAdjTX, tiles_y = (NY + kAdjTY - 1) / kAdjTY;
-  const int tiles_z = (NZ + kAdjTZ - 1) / kAdjTZ;
+  const int tiles_z = (NZ + TZ - 1) / TZ;
   int tile = blockIdx.x;
   const int tx = tile % tiles_x;
   tile /= tiles_x;
@@ -364,26 +367,26 @@ __global__ __launch_bounds__(kAdjThreads) void k_warp_backward(const float* __re
   const int tz = tile % tiles_z;
   const int b = tile / tiles_z;
   const int t = threadIdx.x;
-  const int x = tx * kAdjTX + t % kAdjTX, y = ty * kAdjTY + (t / kAdjTX) % kAdjTY, z = tz * kAdjTZ + t / (kAdjTX * kAdjTY);
-  const bool valid = x < NX && y < NY && z < NZ;
+  const int x = tx * kAdjTX + t % kAdjTX, y = ty * kAdjTY + t / kAdjTX % kAdjTY;
+  const int z1 = x < NX && y < NY ? min(NZ, tz * TZ + TZ) : 0;
   const int64_t N = (int64_t)NZ * NY * NX;
-  const int64_t i = ((int64_t)z * NY + y) * NX + x;
-  float cx = 0.0f, cy = 0.0f, cz = 0.0f;
-  if (valid) {
-    const float* ph = phi + ((int64_t)b * N + i) * 3;
-    cx = (float)x * hX + ph[0];
-    cy = (float)y * hY + ph[1];
-    cz = (float)z * hZ + ph[2];
-  }
-  const int wz0 = tz * kAdjTZ - (kAdjM + 2), wy0 = ty * kAdjTY - (kAdjM + 2), wx0 = tx * kAdjTX - (kAdjM + 2);
-  float gphi[3] = {0.0f, 0.0f, 0.0f};
+  const int wz0 = tz * TZ - (kAdjM + 2), wy0 = ty * kAdjTY - (kAdjM + 2), wx0 = tx * kAdjTX - (kAdjM + 2);
   for (int c = 0; c < C; ++c) {
     const int64_t off = ((int64_t)b * C + c) * N;
-    for (int k = t; k < kAdjWin; k += kAdjThreads) win[k] = 0.0f;
+    for (int k = t; k < kWin; k += kAdjThreads) win[k] = 0.0;
     __syncthreads();
-    if (valid) {
+#pragma unroll 1
+    for (int z = tz * TZ + t / (kAdjTX * kAdjTY); z < z1; z += kAdjG) {
+      const int64_t i = ((int64_t)z * NY + y) * NX + x;
+      const float* ph = phi + ((int64_t)b * N + i) * 3;
+      float* gp = grad_phi + ((int64_t)b * N + i) * 3;
+      const float cx = (float)x * hX + ph[0];
+      const float cy = (float)y * hY + ph[1];
+      const float cz = (float)z * hZ + ph[2];
+      float gphi[3] = {0.0f, 0.0f, 0.0f};
+      if (c > 0) { gphi[0] = gp[0]; gphi[1] = gp[1]; gphi[2] = gp[2]; }
       const float fv = gout[off + i];
-      const WindowAcc acc{win, wz0, wy0, wx0, GlobalAcc{grad_u + off, NY, NX}};
+      const WindowAcc<kWZ> acc{(LdsDouble)win, wz0, wy0, wx0, GlobalAcc{grad_u + off, NY, NX}};
       if (ip == IP_CUBIC) {
         warp_backward_cubic(u + off, acc, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, fv, gphi);
       } else if (ip == IP_LINEAR) {
@@ -391,24 +394,21 @@ __global__ __launch_bounds__(kAdjThreads) void k_warp_backward(const float* __re
       } else {
         acc(nearest_axis(cz, hZ, NZ, bc), nearest_axis(cy, hY, NY, bc), nearest_axis(cx, hX, NX, bc), fv);
       }
+      gp[0] = gphi[0];
+      gp[1] = gphi[1];
+      gp[2] = gphi[2];
     }
     __syncthreads();
     // Only in-volume cells ever receive a contribution (taps are mapped into
     // the volume first), so a non-zero cell is always a valid voxel.
-    for (int k = t; k < kAdjWin; k += kAdjThreads) {
-      const float v = win[k];
+    for (int k = t; k < kWin; k += kAdjThreads) {
+      const float v = (float)win[k];
       if (v != 0.0f) {
         const int lx = k % kAdjWX, ly = (k / kAdjWX) % kAdjWY, lz = k / (kAdjWX * kAdjWY);
         unsafeAtomicAdd(grad_u + off + ((int64_t)(wz0 + lz) * NY + (wy0 + ly)) * NX + (wx0 + lx), v);
       }
     }
     __syncthreads();
-  }
-  if (valid) {
-    float* gp = grad_phi + ((int64_t)b * N + i) * 3;
-    gp[0] = gphi[0];
-    gp[1] = gphi[1];
-    gp[2] = gphi[2];
   }
 }
 
@@ -720,11 +720,18 @@ int svs_warp3d_backward(const float* u, const float* phi, const float* grad_out,
   const int64_t n = (int64_t)NZ * NY * NX;
   int rc = launch_fill(grad_u, (int64_t)B * C * n, 0.0f, (hipStream_t)stream);
   if (rc) return rc;
-  const int64_t tiles = (int64_t)B * ((NX + kAdjTX - 1) / kAdjTX) * ((NY + kAdjTY - 1) / kAdjTY) *
-                        ((NZ + kAdjTZ - 1) / kAdjTZ);
+  const int64_t columns = (int64_t)B * ((NX + kAdjTX - 1) / kAdjTX) * ((NY + kAdjTY - 1) / kAdjTY);
+  // Tiles of 4 planes where they are more than the device runs at once (2 on
+  // each of 256 CUs): fewer window cells per voxel, 2 x 2 x 80^3 (1000 tiles) 180 us
+  // against 182, 4 x 4 x 80^3 643 against 681.  Of 2 planes below, where the
+  // column's length is the time: 64^3 (256 tiles) 31 us against 36, 24^3 21 against
+  // 36, 80^3 (500 tiles) 52 against 53.
+  const int tz = columns * ((NZ + 3) / 4) > 512 ? 4 : 2;
+  const int64_t tiles = columns * ((NZ + tz - 1) / tz);
   SVS_REQUIRE(tiles < ((int64_t)1 << 31), "Warping3D.backward: too many tiles");
-  k_warp_backward<<<(int)tiles, kAdjThreads, 0, (hipStream_t)stream>>>(u, phi, grad_out, B, C, NZ, NY, NX, hZ, hY,
-                                                                       hX, interp, bdry, grad_u, grad_phi);
+  const auto kernel = tz == 4 ? k_warp_backward<4> : k_warp_backward<2>;
+  kernel<<<(int)tiles, kAdjThreads, 0, (hipStream_t)stream>>>(u, phi, grad_out, B, C, NZ, NY, NX, hZ, hY, hX, interp,
+                                                              bdry, grad_u, grad_phi);
   SVS_LAUNCHED();
   return SVS_STATUS_OK;
 }
