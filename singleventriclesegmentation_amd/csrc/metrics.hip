@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kMetricBlock) void k_mask_edges(const float* __rest
   const int64_t i = (int64_t)blockIdx.x * kMetricBlock + threadIdx.x;
   if (i >= (int64_t)NZ * NY * NX) return;
   int z, y, x;
-  unflatten(i, NY, NX, z, y, x);
+  unflatten((unsigned)i, NY, NX, z, y, x);
   if (!(m[i] > 0.5f)) return;
   const bool inner = mask_at(m, z - 1, y, x, NZ, NY, NX) && mask_at(m, z + 1, y, x, NZ, NY, NX) &&
                      mask_at(m, z, y - 1, x, NZ, NY, NX) && mask_at(m, z, y + 1, x, NZ, NY, NX) &&
@@ -96,7 +96,7 @@ __global__ __launch_bounds__(kMetricBlock) void k_directed_hausdorff2(
   int az = 0, ay = 0, ax = 0;
   if (active) {
     int z, y, x;
-    unflatten((int64_t)ea[i], NY, NX, z, y, x);
+    unflatten(ea[i], NY, NX, z, y, x);
     az = z; ay = y; ax = x;
   }
   unsigned long long best = ~0ull;
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(kMetricBlock) void k_directed_hausdorff2(
     const unsigned long long j = base + threadIdx.x;
     if (j < nb) {
       int z, y, x;
-      unflatten((int64_t)eb[j], NY, NX, z, y, x);
+      unflatten(eb[j], NY, NX, z, y, x);
       tz[threadIdx.x] = z; ty[threadIdx.x] = y; tx[threadIdx.x] = x;
     }
     __syncthreads();

@@ -12,6 +12,8 @@
 
 #include <string.h>
 
+#include <algorithm>
+
 namespace svs {
 
 thread_local char g_last_error[1024] = "";
@@ -40,7 +42,7 @@ __global__ __launch_bounds__(kBlock) void k_nabla_fwd(const float* __restrict__ 
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= (int64_t)NZ * NY * NX) return;
   int z, y, x;
-  unflatten(i, NY, NX, z, y, x);
+  unflatten((unsigned)i, NY, NX, z, y, x);
   const int64_t sx = C, sy = (int64_t)NX * C, sz = (int64_t)NY * NX * C;
   for (int c = 0; c < C; ++c) {
     const float* p = b + i * C + c;
@@ -62,7 +64,7 @@ __global__ __launch_bounds__(kBlock) void k_nabla_bwd(const float* __restrict__ 
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= (int64_t)NZ * NY * NX) return;
   int z, y, x;
-  unflatten(i, NY, NX, z, y, x);
+  unflatten((unsigned)i, NY, NX, z, y, x);
   const int64_t sx = 3 * C, sy = (int64_t)NX * 3 * C, sz = (int64_t)NY * NX * 3 * C;
   for (int c = 0; c < C; ++c) {
     const float* q = p + (i * C + c) * 3;
@@ -143,29 +145,38 @@ __global__ __launch_bounds__(kBlock) void k_prox_dual(const float* __restrict__ 
 }
 
 // ------------------------------------------------------------- warping
-// One strided scalar component of a [Z,Y,X,C] (or [B,C,Z,Y,X]) field.
+// One strided scalar component of a [Z,Y,X,C] (or [B,C,Z,Y,X]) field: value
+// `add` of each voxel's `stride`.  I is the type of its byte offsets: unsigned
+// where the field has that many bytes (narrow), so that a tap's address is a
+// scalar base and a 32-bit lane offset.
+template <class I>
 struct StridedFetch {
   const float* base;
-  int64_t stride;
+  I stride, add;
   int NY, NX;
   __device__ void operator()(int z, int y, int x, float* v) const {
-    v[0] = base[(((int64_t)z * NY + y) * NX + x) * stride];
+    const I at = (I)((z * NY + y) * NX + x) * stride + add;
+    v[0] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + at * (I)sizeof(float));
   }
 };
+static bool narrow(int64_t elements) { return elements < ((int64_t)1 << 30); }
 
 // Warping3D.forward / forwardVectorField (warpingOps.cu:572-596, :632-660):
 // out(i) = u(i*h + phi(i)), u [Z,Y,X,C].
-__global__ __launch_bounds__(kBlock) void k_warp(const float* __restrict__ u, int C, const float* __restrict__ phi, int NZ, int NY,
+// CC is C where it is 1 (taps without a multiplication), else 0.
+template <class I, int CC>
+__global__ __launch_bounds__(kBlock) void k_warp(const float* __restrict__ u, int Cany, const float* __restrict__ phi, int NZ, int NY,
                        int NX, float hZ, float hY, float hX, int ip, int bc, float* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= (int64_t)NZ * NY * NX) return;
+  const int C = CC ? CC : Cany;
   int z, y, x;
-  unflatten(i, NY, NX, z, y, x);
+  unflatten((unsigned)i, NY, NX, z, y, x);
   const float cx = (float)x * hX + phi[3 * i + 0];
   const float cy = (float)y * hY + phi[3 * i + 1];
   const float cz = (float)z * hZ + phi[3 * i + 2];
   for (int c = 0; c < C; ++c) {
-    StridedFetch f{u + c, C, NY, NX};
+    const StridedFetch<I> f{u + c, (I)C, 0, NY, NX};
     float v[1];
     sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
     out[i * C + c] = v[0];
@@ -173,25 +184,29 @@ __global__ __launch_bounds__(kBlock) void k_warp(const float* __restrict__ u, in
 }
 
 // WarpingCNN3D.forward (warpingOpsCNN.cu:97-128): u [B,C,Z,Y,X], phi [B,Z,Y,X,3].
+// One launch row per sample of the batch (rows stride over a larger batch).
+// Bound by the taps' address arithmetic and L1 traffic: 8 x 80^3 linear 53 -> 47 us
+// with 32-bit offsets and without 64-bit divisions.
+template <class I>
 __global__ __launch_bounds__(kBlock) void k_warp_cnn(const float* __restrict__ u, const float* __restrict__ phi, int B, int C, int NZ,
                            int NY, int NX, float hZ, float hY, float hX, int ip, int bc, float* __restrict__ out) {
-  const int64_t N = (int64_t)NZ * NY * NX;
-  const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (t >= (int64_t)B * N) return;
-  const int b = (int)(t / N);
-  const int64_t i = t - (int64_t)b * N;
+  const int N = NZ * NY * NX;
+  const unsigned i = blockIdx.x * (unsigned)kBlock + threadIdx.x;
+  if (i >= (unsigned)N) return;
   int z, y, x;
-  unflatten(i, NY, NX, z, y, x);
-  const float* ph = phi + ((int64_t)b * N + i) * 3;
-  const float cx = (float)x * hX + ph[0];
-  const float cy = (float)y * hY + ph[1];
-  const float cz = (float)z * hZ + ph[2];
-  for (int c = 0; c < C; ++c) {
-    const int64_t off = ((int64_t)b * C + c) * N;
-    StridedFetch f{u + off, 1, NY, NX};
-    float v[1];
-    sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
-    out[off + i] = v[0];
+  unflatten((unsigned)i, NY, NX, z, y, x);
+  for (int b = blockIdx.y; b < B; b += gridDim.y) {
+    const float* ph = phi + (int64_t)b * N * 3 + (int64_t)i * 3;
+    const float cx = (float)x * hX + ph[0];
+    const float cy = (float)y * hY + ph[1];
+    const float cz = (float)z * hZ + ph[2];
+    for (int c = 0; c < C; ++c) {
+      const int64_t off = ((int64_t)b * C + c) * N;
+      const StridedFetch<I> f{u + off, 1, 0, NY, NX};
+      float v[1];
+      sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
+      out[off + i] = v[0];
+    }
   }
 }
 
@@ -415,6 +430,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_warp_backward(const float* __re
 // --------------------------------------------------------- prolongation
 // Prolongation3D.forward / forwardVectorField / forwardMatrixField
 // (prolongationOps.cu:533-625): source coordinate ((i * hP) * L) / LP.
+template <class I>
 __global__ __launch_bounds__(kBlock) void k_prolongate(const float* __restrict__ u, int C, int NZ, int NY, int NX, float LZ, float LY,
                              float LX, float hZ, float hY, float hX, int NZp, int NYp, int NXp, float LZp,
                              float LYp, float LXp, float hZp, float hYp, float hXp, int ip, int bc,
@@ -422,7 +438,7 @@ __global__ __launch_bounds__(kBlock) void k_prolongate(const float* __restrict__
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= (int64_t)NZp * NYp * NXp) return;
   int z, y, x;
-  unflatten(i, NYp, NXp, z, y, x);
+  unflatten((unsigned)i, NYp, NXp, z, y, x);
   const float cxp = (float)x * hXp;
   const float cx = cxp * LX / LXp;
   const float cyp = (float)y * hYp;
@@ -430,10 +446,52 @@ __global__ __launch_bounds__(kBlock) void k_prolongate(const float* __restrict__
   const float czp = (float)z * hZp;
   const float cz = czp * LZ / LZp;
   for (int c = 0; c < C; ++c) {
-    StridedFetch f{u + c, C, NY, NX};
+    const StridedFetch<I> f{u + c, (I)C, 0, NY, NX};
     float v[1];
     sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
     out[i * C + c] = v[0];
+  }
+}
+
+// The same with many channels, a thread per (voxel, channel): lanes run along
+// the channels, so taps and output are read and written in whole lines.  A
+// work-group writes kProlongChunk consecutive values and first splits their
+// voxels' coordinates, each once, into LDS.  25 frames of 12 x 160 x 144 to 80^3,
+// linear: 1.1 ms with a thread per voxel (each tap a line of its own per lane),
+// 69 us like this; what bounds it now is the arithmetic per value (8 weights,
+// their products and addresses).
+constexpr int kProlongChunk = 2048, kProlongChannels = 4;
+template <class I>
+__global__ __launch_bounds__(kBlock) void k_prolongate_field(
+    const float* __restrict__ u, int C, int NZ, int NY, int NX, float LZ, float LY, float LX, float hZ, float hY, float hX,
+    int NZp, int NYp, int NXp, float LZp, float LYp, float LXp, float hZp, float hYp, float hXp, int ip, int bc,
+    float* __restrict__ out) {
+  __shared__ Axis axes[kProlongChunk / kProlongChannels + 2][3];
+  const int64_t first = (int64_t)blockIdx.x * kProlongChunk, n = (int64_t)NZp * NYp * NXp;
+  const int64_t v0 = first / C;
+  const unsigned c0 = (unsigned)(first - v0 * C);
+  const unsigned count = (unsigned)min(n * C - first, (int64_t)kProlongChunk);
+  const unsigned voxels = (c0 + count - 1) / (unsigned)C + 1;
+  for (unsigned k = threadIdx.x; k < voxels; k += kBlock) {
+    int z, y, x;
+    unflatten((unsigned)v0 + k, NYp, NXp, z, y, x);
+    const float cxp = (float)x * hXp;
+    const float cx = cxp * LX / LXp;
+    const float cyp = (float)y * hYp;
+    const float cy = cyp * LY / LYp;
+    const float czp = (float)z * hZp;
+    const float cz = czp * LZ / LZp;
+    axes[k][0] = sample_axis(ip, cx, hX, NX, bc);
+    axes[k][1] = sample_axis(ip, cy, hY, NY, bc);
+    axes[k][2] = sample_axis(ip, cz, hZ, NZ, bc);
+  }
+  __syncthreads();
+  for (unsigned e = threadIdx.x; e < count; e += kBlock) {
+    const unsigned k = (c0 + e) / (unsigned)C, c = c0 + e - k * (unsigned)C;
+    const StridedFetch<I> f{u, (I)C, (I)c, NY, NX};
+    float v[1];
+    sample_at<1>(ip, f, NZ, NY, NX, bc, axes[k][2], axes[k][1], axes[k][0], v);
+    out[first + e] = v[0];
   }
 }
 
@@ -445,7 +503,7 @@ __global__ __launch_bounds__(kBlock) void k_blur(const float* __restrict__ in, i
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= (int64_t)NZ * NY * NX) return;
   int z, y, x;
-  unflatten(i, NY, NX, z, y, x);
+  unflatten((unsigned)i, NY, NX, z, y, x);
   const int P = K / 2;
   float acc = 0.0f;
   for (int a = 0; a < K; ++a) {
@@ -561,7 +619,7 @@ __global__ __launch_bounds__(kBlock) void k_median_any(const float* __restrict__
   const int64_t N = (int64_t)NZ * NY * NX;
   const int64_t b = i / N;
   int z, y, x;
-  unflatten(i - b * N, NY, NX, z, y, x);
+  unflatten((unsigned)(i - b * N), NY, NX, z, y, x);
   const float* src = in + b * N * C + c;
   float win[kMedianMaxK * kMedianMaxK * kMedianMaxK];
   const int h = ks / 2, n = ks * ks * ks;
@@ -690,8 +748,8 @@ int svs_warp3d(const float* u, int C, const float* phi, int NZ, int NY, int NX, 
   SVS_REQUIRE_DIMS(NZ, NY, NX);
   SVS_REQUIRE(valid_bc(bdry) && valid_ip(interp), "Warping3D.forward: invalid interpolation/boundary type");
   const int64_t n = (int64_t)NZ * NY * NX;
-  k_warp<<<grid_for(n, kBlock), kBlock, 0, (hipStream_t)stream>>>(u, C, phi, NZ, NY, NX, hZ, hY, hX, interp, bdry,
-                                                                  out);
+  const auto kernel = !narrow(n * C) ? k_warp<int64_t, 0> : C == 1 ? k_warp<unsigned, 1> : k_warp<unsigned, 0>;
+  kernel<<<grid_for(n, kBlock), kBlock, 0, (hipStream_t)stream>>>(u, C, phi, NZ, NY, NX, hZ, hY, hX, interp, bdry, out);
   SVS_LAUNCHED();
   return SVS_STATUS_OK;
 }
@@ -704,8 +762,10 @@ int svs_warp3d_cnn(const float* u, const float* phi, int B, int C, int NZ, int N
   SVS_REQUIRE(valid_bc(bdry) && valid_ip(interp), "WarpingCNN3D.forward: invalid interpolation/boundary type");
   const int64_t n = (int64_t)B * NZ * NY * NX;
   SVS_REQUIRE_WORKITEMS(n, "WarpingCNN3D.forward (batch x voxels)");
-  k_warp_cnn<<<grid_for(n, kBlock), kBlock, 0, (hipStream_t)stream>>>(u, phi, B, C, NZ, NY, NX, hZ, hY, hX, interp,
-                                                                      bdry, out);
+  const int64_t N = (int64_t)NZ * NY * NX;
+  const auto kernel = narrow(N) ? k_warp_cnn<unsigned> : k_warp_cnn<int64_t>;
+  kernel<<<dim3(grid_for(N, kBlock), std::min(B, 65535)), kBlock, 0, (hipStream_t)stream>>>(
+      u, phi, B, C, NZ, NY, NX, hZ, hY, hX, interp, bdry, out);
   SVS_LAUNCHED();
   return SVS_STATUS_OK;
 }
@@ -746,9 +806,15 @@ int svs_prolongate3d(const float* u, int C, int NZ, int NY, int NX, float LZ, fl
   const float hZ = LZ / (float)(NZ - 1), hY = LY / (float)(NY - 1), hX = LX / (float)(NX - 1);
   const float hZp = LZp / (float)(NZp - 1), hYp = LYp / (float)(NYp - 1), hXp = LXp / (float)(NXp - 1);
   const int64_t n = (int64_t)NZp * NYp * NXp;
-  k_prolongate<<<grid_for(n, kBlock), kBlock, 0, (hipStream_t)stream>>>(u, C, NZ, NY, NX, LZ, LY, LX, hZ, hY, hX,
-                                                                        NZp, NYp, NXp, LZp, LYp, LXp, hZp, hYp,
-                                                                        hXp, interp, bdry, out);
+  const bool lean = narrow((int64_t)NZ * NY * NX * C);
+  const int64_t chunks = (n * C + kProlongChunk - 1) / kProlongChunk;
+  // A thread per voxel for few channels: nothing is gained by sharing a
+  // coordinate among lanes there, and the table would outgrow the LDS.
+  const bool field = C >= kProlongChannels && chunks < ((int64_t)1 << 31);
+  const auto kernel = field ? (lean ? k_prolongate_field<unsigned> : k_prolongate_field<int64_t>)
+                            : (lean ? k_prolongate<unsigned> : k_prolongate<int64_t>);
+  kernel<<<field ? (int)chunks : grid_for(n, kBlock), kBlock, 0, (hipStream_t)stream>>>(
+      u, C, NZ, NY, NX, LZ, LY, LX, hZ, hY, hX, NZp, NYp, NXp, LZp, LYp, LXp, hZp, hYp, hXp, interp, bdry, out);
   SVS_LAUNCHED();
   return SVS_STATUS_OK;
 }

@@ -98,7 +98,7 @@ __device__ __forceinline__ int find_instance(const int* __restrict__ block_start
   const int64_t i = (int64_t)(blockIdx.x - block_start[inst_]) * kBlock + threadIdx.x; \
   if (i >= d.N) return;                                                            \
   int z, y, x;                                                                     \
-  unflatten(i, d.NY, d.NX, z, y, x)
+  unflatten((unsigned)i, d.NY, d.NX, z, y, x)
 
 // ---------------------------------------------------------- level set-up
 // Gaussian pre-blur of both frames of every instance (flow_utils.py:94-112).

@@ -253,6 +253,20 @@ __device__ __forceinline__ int nearest_axis(float coord, float h, int N, int bc)
   return dist_f < dist_c ? bidx(f, N, bc) : bidx(f + 1, N, bc);
 }
 
+// The sample at a coordinate already split per axis; for IP_NEAREST, f is the
+// voxel itself (nearest_axis).
+__device__ __forceinline__ Axis sample_axis(int ip, float coord, float h, int N, int bc) {
+  if (ip != IP_NEAREST) return make_axis(coord, h);
+  return Axis{nearest_axis(coord, h, N, bc), 0.0f};
+}
+template <int NC, class Fetch>
+__device__ __forceinline__ void sample_at(int ip, const Fetch& fetch, int NZ, int NY, int NX, int bc, Axis az, Axis ay,
+                                          Axis ax, float out[NC]) {
+  if (ip == IP_CUBIC) sample_cubic<NC>(fetch, NZ, NY, NX, az, ay, ax, bc, out);
+  else if (ip == IP_LINEAR) sample_linear<NC>(fetch, NZ, NY, NX, az, ay, ax, bc, out);
+  else fetch(az.f, ay.f, ax.f, out);
+}
+
 template <int NC, class Fetch, int LOOP = 0>
 __device__ __forceinline__ void sample(int ip, const Fetch& fetch, int NZ, int NY, int NX, float hZ, float hY,
                                        float hX, int bc, float cz, float cy, float cx, float out[NC]) {
@@ -437,12 +451,14 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Linear voxel index -> (z, y, x).
-__device__ __forceinline__ void unflatten(int64_t i, int NY, int NX, int& z, int& y, int& x) {
-  x = (int)(i % NX);
-  const int64_t t = i / NX;
-  y = (int)(t % NY);
-  z = (int)(t / NY);
+// Linear voxel index (a volume has fewer than 2^32 voxels: a 64-bit division
+// by a variable costs some 100 instructions, four of them per voxel) ->
+// (z, y, x).
+__device__ __forceinline__ void unflatten(unsigned i, int NY, int NX, int& z, int& y, int& x) {
+  const unsigned t = i / (unsigned)NX;
+  x = (int)(i - t * (unsigned)NX);
+  z = (int)(t / (unsigned)NY);
+  y = (int)(t - (unsigned)z * (unsigned)NY);
 }
 
 }  // namespace svs
