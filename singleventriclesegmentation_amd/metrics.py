@@ -32,11 +32,16 @@ def _mask3d(t: torch.Tensor, name: str) -> torch.Tensor:
     return t.contiguous()
 
 
-def mask_counts(y_pred: torch.Tensor, y: torch.Tensor) -> Tuple[int, int, int]:
-    """(|pred|, |gt|, |pred and gt|) of two binary masks (value > 0.5 is set)."""
+def _pair(y_pred, y):
     a, b = _mask3d(y_pred, "y_pred"), _mask3d(y, "y")
     if a.shape != b.shape or a.device != b.device:
         raise RuntimeError("masks must have the same shape and device")
+    return a, b
+
+
+def mask_counts(y_pred: torch.Tensor, y: torch.Tensor) -> Tuple[int, int, int]:
+    """(|pred|, |gt|, |pred and gt|) of two binary masks (value > 0.5 is set)."""
+    a, b = _pair(y_pred, y)
     with torch.cuda.device(a.device):
         out = torch.empty(3, dtype=torch.int64, device=a.device)
         check(_lib.lib().svs_mask_counts(ptr(a), ptr(b), *a.shape, ptr(out), stream_ptr()))
@@ -44,37 +49,51 @@ def mask_counts(y_pred: torch.Tensor, y: torch.Tensor) -> Tuple[int, int, int]:
     return c[0], c[1], c[2]
 
 
-def compute_dice(y_pred: torch.Tensor, y: torch.Tensor) -> float:
-    """monai compute_dice(y_pred, y, include_background=False) on one binary channel."""
-    na, nb, nab = mask_counts(y_pred, y)
+def _dice(na, nb, nab):
     if nb == 0:
         return float("nan")
     return float(np.float32(2.0 * nab) / np.float32(na + nb))
 
 
+def compute_dice(y_pred: torch.Tensor, y: torch.Tensor) -> float:
+    """monai compute_dice(y_pred, y, include_background=False) on one binary channel."""
+    return _dice(*mask_counts(y_pred, y))
+
+
+# The workspace of svs_mask_hausdorff2 begins with 8 words: the call writes the
+# edge counts to the first two, the next two take its distances and three more
+# the voxel counts, so that one copy brings a pair's results to the host.
+_HEADER = 8
+
+
+def _workspace_words(a):
+    return (_lib.lib().svs_mask_hausdorff_workspace_bytes(*a.shape) + 7) // 8
+
+
+def _enqueue_hausdorff(a, b, ws):
+    check(_lib.lib().svs_mask_hausdorff2(ptr(a), ptr(b), *a.shape, ptr(ws), ws.numel() * 8, ptr(ws[2:4]), stream_ptr()))
+
+
 def directed_hausdorff2(y_pred: torch.Tensor, y: torch.Tensor) -> Tuple[int, int, int, int]:
     """(d2 pred->gt, d2 gt->pred, edge voxels of pred, edge voxels of gt)."""
-    a, b = _mask3d(y_pred, "y_pred"), _mask3d(y, "y")
-    if a.shape != b.shape or a.device != b.device:
-        raise RuntimeError("masks must have the same shape and device")
-    lib = _lib.lib()
-    nbytes = lib.svs_mask_hausdorff_workspace_bytes(*a.shape)
+    a, b = _pair(y_pred, y)
     with torch.cuda.device(a.device):
-        ws = torch.empty((nbytes + 7) // 8, dtype=torch.int64, device=a.device)
-        out = torch.empty(2, dtype=torch.int64, device=a.device)
-        check(lib.svs_mask_hausdorff2(ptr(a), ptr(b), *a.shape, ptr(ws), ws.numel() * 8, ptr(out), stream_ptr()))
-        d = out.cpu().tolist()
-        e = ws[:2].cpu().tolist()
-    return d[0], d[1], e[0], e[1]
+        ws = torch.empty(_workspace_words(a), dtype=torch.int64, device=a.device)
+        _enqueue_hausdorff(a, b, ws)
+        ea, eb, d_ab, d_ba = ws[:4].cpu().tolist()
+    return d_ab, d_ba, ea, eb
+
+
+def _hausdorff(d_ab, d_ba, ea, eb):
+    if ea == 0 or eb == 0:
+        return float("nan")
+    return float(np.float32(math.sqrt(float(max(d_ab, d_ba)))))
 
 
 def compute_hausdorff_distance(y_pred: torch.Tensor, y: torch.Tensor) -> float:
     """monai compute_hausdorff_distance(y_pred, y, include_background=False)
     (Euclidean, symmetric, no percentile) on one binary channel."""
-    d_ab, d_ba, ea, eb = directed_hausdorff2(y_pred, y)
-    if ea == 0 or eb == 0:
-        return float("nan")
-    return float(np.float32(math.sqrt(float(max(d_ab, d_ba)))))
+    return _hausdorff(*directed_hausdorff2(y_pred, y))
 
 
 def propagation_metrics(forward_masks: torch.Tensor, backward_masks: torch.Tensor):
@@ -82,5 +101,19 @@ def propagation_metrics(forward_masks: torch.Tensor, backward_masks: torch.Tenso
     returns (dice_bwd, dice_fwd, hausdorff_bwd, hausdorff_fwd)."""
     initial_gt, initial_pred = forward_masks[0], backward_masks[0]
     final_gt, final_pred = backward_masks[-1], forward_masks[-1]
-    return (compute_dice(initial_pred, initial_gt), compute_dice(final_pred, final_gt),
-            compute_hausdorff_distance(initial_pred, initial_gt), compute_hausdorff_distance(final_pred, final_gt))
+    pairs = [_pair(initial_pred, initial_gt), _pair(final_pred, final_gt)]
+    same = pairs[0][0].shape == pairs[1][0].shape and pairs[0][0].device == pairs[1][0].device
+    if not same:
+        return (compute_dice(initial_pred, initial_gt), compute_dice(final_pred, final_gt),
+                compute_hausdorff_distance(initial_pred, initial_gt), compute_hausdorff_distance(final_pred, final_gt))
+    # Both pairs' work is enqueued before the one copy that waits for it.
+    a = pairs[0][0]
+    with torch.cuda.device(a.device):
+        ws = torch.empty((2, _workspace_words(a)), dtype=torch.int64, device=a.device)
+        for (x, y), w in zip(pairs, ws):
+            check(_lib.lib().svs_mask_counts(ptr(x), ptr(y), *x.shape, ptr(w[4:7]), stream_ptr()))
+            _enqueue_hausdorff(x, y, w)
+        words = ws[:, :_HEADER].cpu().tolist()
+    dice = [_dice(*w[4:7]) for w in words]
+    distance = [_hausdorff(w[2], w[3], w[0], w[1]) for w in words]
+    return (*dice, *distance)
