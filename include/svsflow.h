@@ -84,6 +84,16 @@ int svs_warp3d(const float* u, int C, const float* phi, int NZ, int NY, int NX, 
 int svs_warp3d_cnn(const float* u, const float* phi, int B, int C, int NZ, int NY, int NX, float hZ, float hY,
                    float hX, int interpolation, int bdry, float* out, void* stream);
 
+/* Both chains of the mask propagation (OpticalFlowWarper._propagate,
+ * warping.py:205-243).  Masks [C,Z,Y,X]; step t of a chain warps by the flow
+ * [Z,Y,X,3] at flow + t * stride floats.  out_fwd and out_bwd [T+1,C,Z,Y,X]
+ * receive every continuous mask thresholded (value > threshold) to 0 or 1, the
+ * backward chain's in reverse.  scratch: 4 masks' floats. */
+int svs_propagate_masks(const float* mask_fwd, const float* mask_bwd, const float* flow_fwd, int64_t stride_fwd,
+                        const float* flow_bwd, int64_t stride_bwd, int T, int C, int NZ, int NY, int NX, float hZ, float hY,
+                        float hX, int interpolation, int bdry, float threshold, float* scratch, float* out_fwd,
+                        float* out_bwd, void* stream);
+
 /* Adjoint of the warp with respect to the warped volume and the flow.
  * B = C = 1 is Warping3D.backward(u, phi, grad_out) -> [grad_u, grad_phi]
  * (warpingOps.h:98-103, warpingOps.cu:1173); B, C > 1 is the batched CNN form

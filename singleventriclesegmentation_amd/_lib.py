@@ -58,6 +58,8 @@ _SIGNATURES = {
     "svs_prox_primal": ([_vp, _f, _f, _vp, _vp, _i64, _vp, _vp], _i),
     "svs_prox_dual": ([_vp, _f, _f, _i64, _vp, _vp], _i),
     "svs_warp3d": ([_vp, _i, _vp, _i, _i, _i, _f, _f, _f, _i, _i, _vp, _vp], _i),
+    "svs_propagate_masks": ([_vp, _vp, _vp, ctypes.c_int64, _vp, ctypes.c_int64, _i, _i, _i, _i, _i, _f, _f, _f, _i, _i, _f,
+                             _vp, _vp, _vp, _vp], _i),
     "svs_warp3d_cnn": ([_vp, _vp, _i, _i, _i, _i, _i, _f, _f, _f, _i, _i, _vp, _vp], _i),
     "svs_warp3d_backward": ([_vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _f, _f, _i, _i, _vp, _vp, _vp], _i),
     "svs_prolongate3d": ([_vp, _i, _i, _i, _i, _f, _f, _f, _i, _i, _i, _f, _f, _f, _i, _i, _vp, _vp], _i),

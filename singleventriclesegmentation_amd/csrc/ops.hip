@@ -210,6 +210,42 @@ __global__ __launch_bounds__(kBlock) void k_warp_cnn(const float* __restrict__ u
   }
 }
 
+// One step of both mask chains (OpticalFlowWarper._propagate,
+// warping.py:205-243): row y of the launch warps chain y's continuous masks
+// with k_warp_cnn's arithmetic and writes them for the next step (unless this is
+// the last) and thresholded to their place in the result.  The first step also
+// thresholds the masks it starts from.
+struct ChainStep {
+  const float* in;
+  const float* phi;
+  float* out;         // null: last step
+  float* set;         // thresholded output
+  float* set_first;   // null: not the first step
+};
+template <class I>
+__global__ __launch_bounds__(kBlock) void k_propagate(ChainStep fwd, ChainStep bwd, int C, int NZ, int NY, int NX, float hZ,
+                                                      float hY, float hX, int ip, int bc, float threshold) {
+  const int N = NZ * NY * NX;
+  const unsigned i = blockIdx.x * (unsigned)kBlock + threadIdx.x;
+  if (i >= (unsigned)N) return;
+  const ChainStep s = blockIdx.y ? bwd : fwd;
+  int z, y, x;
+  unflatten(i, NY, NX, z, y, x);
+  const float* ph = s.phi + (int64_t)i * 3;
+  const float cx = (float)x * hX + ph[0];
+  const float cy = (float)y * hY + ph[1];
+  const float cz = (float)z * hZ + ph[2];
+  for (int c = 0; c < C; ++c) {
+    const int64_t off = (int64_t)c * N;
+    const StridedFetch<I> f{s.in + off, 1, 0, NY, NX};
+    float v[1];
+    sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
+    if (s.out) s.out[off + i] = v[0];
+    s.set[off + i] = v[0] > threshold ? 1.0f : 0.0f;
+    if (s.set_first) s.set_first[off + i] = s.in[off + i] > threshold ? 1.0f : 0.0f;
+  }
+}
+
 // Adjoint of one tricubic sample (interpolation_cubicHermiteSpline.cuh:527-636):
 // scatters fwd * d out/d u into grad (atomics, 64 taps) and adds the three
 // flow derivatives to gphi in the reference's order (z, y per dz, x per dy).
@@ -767,6 +803,31 @@ int svs_warp3d_cnn(const float* u, const float* phi, int B, int C, int NZ, int N
   kernel<<<dim3(grid_for(N, kBlock), std::min(B, 65535)), kBlock, 0, (hipStream_t)stream>>>(
       u, phi, B, C, NZ, NY, NX, hZ, hY, hX, interp, bdry, out);
   SVS_LAUNCHED();
+  return SVS_STATUS_OK;
+}
+
+int svs_propagate_masks(const float* mask_fwd, const float* mask_bwd, const float* flow_fwd, int64_t stride_fwd,
+                        const float* flow_bwd, int64_t stride_bwd, int T, int C, int NZ, int NY, int NX, float hZ, float hY,
+                        float hX, int interp, int bdry, float threshold, float* scratch, float* out_fwd, float* out_bwd,
+                        void* stream) {
+  SVS_REQUIRE(mask_fwd && mask_bwd && flow_fwd && flow_bwd && scratch && out_fwd && out_bwd,
+              "mask propagation: null pointer");
+  SVS_REQUIRE(T >= 1 && C >= 1, "mask propagation: steps and channels must be >= 1");
+  SVS_REQUIRE_DIMS(NZ, NY, NX);
+  SVS_REQUIRE(valid_bc(bdry) && valid_ip(interp), "mask propagation: invalid interpolation/boundary type");
+  const int64_t N = (int64_t)NZ * NY * NX, M = N * C;
+  const auto kernel = narrow(N) ? k_propagate<unsigned> : k_propagate<int64_t>;
+  for (int t = 0; t < T; ++t) {
+    const int to = t & 1, from = to ^ 1;
+    ChainStep f{t ? scratch + (2 * from) * M : mask_fwd, flow_fwd + t * stride_fwd,
+                t + 1 < T ? scratch + (2 * to) * M : nullptr, out_fwd + (int64_t)(t + 1) * M, t ? nullptr : out_fwd};
+    ChainStep b{t ? scratch + (2 * from + 1) * M : mask_bwd, flow_bwd + t * stride_bwd,
+                t + 1 < T ? scratch + (2 * to + 1) * M : nullptr, out_bwd + (int64_t)(T - 1 - t) * M,
+                t ? nullptr : out_bwd + (int64_t)T * M};
+    kernel<<<dim3(grid_for(N, kBlock), 2), kBlock, 0, (hipStream_t)stream>>>(f, b, C, NZ, NY, NX, hZ, hY, hX, interp, bdry,
+                                                                           threshold);
+    SVS_LAUNCHED();
+  }
   return SVS_STATUS_OK;
 }
 

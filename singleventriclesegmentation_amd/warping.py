@@ -7,7 +7,8 @@ from typing import Tuple
 
 import torch
 
-from . import opticalFlow
+from . import _lib, opticalFlow
+from ._lib import check, on_device, ptr, stream_ptr
 from .flow_utils import get_interpolation_type, get_mesh_length
 
 
@@ -30,6 +31,39 @@ class Warp:
         return self.op(x).forward(x.contiguous(), u.contiguous())
 
 
+def _plain(t, shape):
+    return type(t) is torch.Tensor and t.is_cuda and t.dtype is torch.float32 and tuple(t.shape) == shape
+
+
+def _propagate_natively(warp, initial_mask, final_mask, forward_flow, backward_flow, threshold):
+    """Both chains in one native call, a launch per step, or None where the
+    arguments are not what it takes (another warp, mixed devices or sizes,
+    flows whose steps are not contiguous, ...)."""
+    if type(warp) is not Warp or type(threshold) not in (int, float) or abs(threshold) > 2 ** 24:
+        return None
+    if type(forward_flow) is not torch.Tensor or forward_flow.dim() != 5 or forward_flow.shape[0] < 1:
+        return None
+    T, NZ, NY, NX = forward_flow.shape[:4]
+    if type(initial_mask) is not torch.Tensor or initial_mask.dim() != 5 or initial_mask.shape[0] != 1 or initial_mask.shape[1] < 1:
+        return None
+    C = initial_mask.shape[1]
+    masks, flows = (initial_mask, final_mask), (forward_flow, backward_flow)
+    if not all(_plain(m, (1, C, NZ, NY, NX)) and m.is_contiguous() for m in masks):
+        return None
+    if not all(_plain(f, (T, NZ, NY, NX, 3)) and f[0].is_contiguous() for f in flows):
+        return None
+    if any(t.device != initial_mask.device for t in (final_mask, forward_flow, backward_flow)):
+        return None
+    op = warp.op(initial_mask)
+    with on_device(initial_mask.device):
+        fwd, bwd = (initial_mask.new_empty((T + 1, C, NZ, NY, NX)) for _ in range(2))
+        scratch = initial_mask.new_empty((4, C, NZ, NY, NX))
+        check(_lib.lib().svs_propagate_masks(
+            *(ptr(m) for m in masks), ptr(forward_flow), forward_flow.stride(0), ptr(backward_flow), backward_flow.stride(0),
+            T, C, NZ, NY, NX, *op._h, op._ip, op._bc, threshold, ptr(scratch), ptr(fwd), ptr(bwd), stream_ptr()))
+    return fwd, bwd
+
+
 def propagate(warp: Warp, initial_mask: torch.Tensor, final_mask: torch.Tensor, forward_flow: torch.Tensor,
               backward_flow: torch.Tensor, threshold: float = 0.5):
     """Mask propagation of OpticalFlowWarper._propagate (warping.py:205-243).
@@ -40,6 +74,9 @@ def propagate(warp: Warp, initial_mask: torch.Tensor, final_mask: torch.Tensor, 
     (forward_masks, backward_masks), each [T+1,1,Z,Y,X] in {0, 1}, the
     backward chain reversed so index 0 is the estimate of the initial mask."""
     assert forward_flow.shape[0] == backward_flow.shape[0], "Forward and backward flow have different timesteps"
+    done = _propagate_natively(warp, initial_mask, final_mask, forward_flow, backward_flow, threshold)
+    if done is not None:
+        return done
     fwd = [initial_mask]
     bwd = [final_mask]
     for t in range(forward_flow.shape[0]):
