@@ -159,37 +159,62 @@ struct StridedFetch {
     v[0] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + at * (I)sizeof(float));
   }
 };
+// One sample of a volume of its own.
+template <class I, int IP>
+__device__ __forceinline__ float sample_unit(const float* u, int NZ, int NY, int NX, float hZ, float hY, float hX, int bc,
+                                             float cz, float cy, float cx) {
+  const StridedFetch<I> f{u, 1, 0, NY, NX};
+  float v[1];
+  sample<1>(IP, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
+  return v[0];
+}
 static bool narrow(int64_t elements) { return elements < ((int64_t)1 << 30); }
+// The instantiation of a kernel template <class I, int IP> for an offset type
+// and an interpolation; each of its own, as the tricubic one's registers would
+// halve the others' waves (k_warp_cnn).
+#define SVS_PICK(kernel, lean, ip)                                                                             \
+  ((lean) ? ((ip) == IP_CUBIC    ? kernel<unsigned, IP_CUBIC>                                                  \
+             : (ip) == IP_LINEAR ? kernel<unsigned, IP_LINEAR>                                                 \
+                                 : kernel<unsigned, IP_NEAREST>)                                               \
+          : ((ip) == IP_CUBIC    ? kernel<int64_t, IP_CUBIC>                                                   \
+             : (ip) == IP_LINEAR ? kernel<int64_t, IP_LINEAR>                                                  \
+                                 : kernel<int64_t, IP_NEAREST>))
 
 // Warping3D.forward / forwardVectorField (warpingOps.cu:572-596, :632-660):
 // out(i) = u(i*h + phi(i)), u [Z,Y,X,C].
-// CC is C where it is 1 (taps without a multiplication), else 0.
-template <class I, int CC>
-__global__ __launch_bounds__(kBlock) void k_warp(const float* __restrict__ u, int Cany, const float* __restrict__ phi, int NZ, int NY,
-                       int NX, float hZ, float hY, float hX, int ip, int bc, float* __restrict__ out) {
+template <class I, int IP>
+__global__ __launch_bounds__(kBlock) void k_warp(const float* __restrict__ u, int C, const float* __restrict__ phi, int NZ, int NY,
+                       int NX, float hZ, float hY, float hX, int bc, float* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= (int64_t)NZ * NY * NX) return;
-  const int C = CC ? CC : Cany;
   int z, y, x;
   unflatten((unsigned)i, NY, NX, z, y, x);
   const float cx = (float)x * hX + phi[3 * i + 0];
   const float cy = (float)y * hY + phi[3 * i + 1];
   const float cz = (float)z * hZ + phi[3 * i + 2];
+  if (C == 1) {
+    out[i] = sample_unit<I, IP>(u, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx);
+    return;
+  }
   for (int c = 0; c < C; ++c) {
     const StridedFetch<I> f{u + c, (I)C, 0, NY, NX};
     float v[1];
-    sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
+    sample<1>(IP, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
     out[i * C + c] = v[0];
   }
 }
 
 // WarpingCNN3D.forward (warpingOpsCNN.cu:97-128): u [B,C,Z,Y,X], phi [B,Z,Y,X,3].
 // One launch row per sample of the batch (rows stride over a larger batch).
-// Bound by the taps' address arithmetic and L1 traffic: 8 x 80^3 linear 53 -> 47 us
-// with 32-bit offsets and without 64-bit divisions.
-template <class I>
+// Linear, 8 x 80^3: 53 us at first, 47 with 32-bit offsets and without 64-bit
+// divisions, 25 with the tricubic case in a kernel of its own (52 registers
+// instead of 123); bound by the taps' passes of the vector memory unit.  Tricubic, 16
+// x 80^3: 151 us, 2700 clocks per wavefront of which some 1200 are the 21
+// segments' arithmetic.  (Rows as unaligned 16-byte loads took twice the time;
+// the taps' box staged in LDS 130 us, but 13 against 6 us for 24^3.)
+template <class I, int IP>
 __global__ __launch_bounds__(kBlock) void k_warp_cnn(const float* __restrict__ u, const float* __restrict__ phi, int B, int C, int NZ,
-                           int NY, int NX, float hZ, float hY, float hX, int ip, int bc, float* __restrict__ out) {
+                           int NY, int NX, float hZ, float hY, float hX, int bc, float* __restrict__ out) {
   const int N = NZ * NY * NX;
   const unsigned i = blockIdx.x * (unsigned)kBlock + threadIdx.x;
   if (i >= (unsigned)N) return;
@@ -202,10 +227,7 @@ __global__ __launch_bounds__(kBlock) void k_warp_cnn(const float* __restrict__ u
     const float cz = (float)z * hZ + ph[2];
     for (int c = 0; c < C; ++c) {
       const int64_t off = ((int64_t)b * C + c) * N;
-      const StridedFetch<I> f{u + off, 1, 0, NY, NX};
-      float v[1];
-      sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
-      out[off + i] = v[0];
+      out[off + i] = sample_unit<I, IP>(u + off, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx);
     }
   }
 }
@@ -222,9 +244,9 @@ struct ChainStep {
   float* set;         // thresholded output
   float* set_first;   // null: not the first step
 };
-template <class I>
+template <class I, int IP>
 __global__ __launch_bounds__(kBlock) void k_propagate(ChainStep fwd, ChainStep bwd, int C, int NZ, int NY, int NX, float hZ,
-                                                      float hY, float hX, int ip, int bc, float threshold) {
+                                                      float hY, float hX, int bc, float threshold) {
   const int N = NZ * NY * NX;
   const unsigned i = blockIdx.x * (unsigned)kBlock + threadIdx.x;
   if (i >= (unsigned)N) return;
@@ -237,11 +259,9 @@ __global__ __launch_bounds__(kBlock) void k_propagate(ChainStep fwd, ChainStep b
   const float cz = (float)z * hZ + ph[2];
   for (int c = 0; c < C; ++c) {
     const int64_t off = (int64_t)c * N;
-    const StridedFetch<I> f{s.in + off, 1, 0, NY, NX};
-    float v[1];
-    sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
-    if (s.out) s.out[off + i] = v[0];
-    s.set[off + i] = v[0] > threshold ? 1.0f : 0.0f;
+    const float v = sample_unit<I, IP>(s.in + off, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx);
+    if (s.out) s.out[off + i] = v;
+    s.set[off + i] = v > threshold ? 1.0f : 0.0f;
     if (s.set_first) s.set_first[off + i] = s.in[off + i] > threshold ? 1.0f : 0.0f;
   }
 }
@@ -466,10 +486,10 @@ __global__ __launch_bounds__(kAdjThreads) void k_warp_backward(const float* __re
 // --------------------------------------------------------- prolongation
 // Prolongation3D.forward / forwardVectorField / forwardMatrixField
 // (prolongationOps.cu:533-625): source coordinate ((i * hP) * L) / LP.
-template <class I>
+template <class I, int IP>
 __global__ __launch_bounds__(kBlock) void k_prolongate(const float* __restrict__ u, int C, int NZ, int NY, int NX, float LZ, float LY,
                              float LX, float hZ, float hY, float hX, int NZp, int NYp, int NXp, float LZp,
-                             float LYp, float LXp, float hZp, float hYp, float hXp, int ip, int bc,
+                             float LYp, float LXp, float hZp, float hYp, float hXp, int bc,
                              float* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= (int64_t)NZp * NYp * NXp) return;
@@ -484,7 +504,7 @@ __global__ __launch_bounds__(kBlock) void k_prolongate(const float* __restrict__
   for (int c = 0; c < C; ++c) {
     const StridedFetch<I> f{u + c, (I)C, 0, NY, NX};
     float v[1];
-    sample<1>(ip, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
+    sample<1>(IP, f, NZ, NY, NX, hZ, hY, hX, bc, cz, cy, cx, v);
     out[i * C + c] = v[0];
   }
 }
@@ -497,10 +517,10 @@ __global__ __launch_bounds__(kBlock) void k_prolongate(const float* __restrict__
 // 69 us like this; what bounds it now is the arithmetic per value (8 weights,
 // their products and addresses).
 constexpr int kProlongChunk = 2048, kProlongChannels = 4;
-template <class I>
+template <class I, int IP>
 __global__ __launch_bounds__(kBlock) void k_prolongate_field(
     const float* __restrict__ u, int C, int NZ, int NY, int NX, float LZ, float LY, float LX, float hZ, float hY, float hX,
-    int NZp, int NYp, int NXp, float LZp, float LYp, float LXp, float hZp, float hYp, float hXp, int ip, int bc,
+    int NZp, int NYp, int NXp, float LZp, float LYp, float LXp, float hZp, float hYp, float hXp, int bc,
     float* __restrict__ out) {
   __shared__ Axis axes[kProlongChunk / kProlongChannels + 2][3];
   const int64_t first = (int64_t)blockIdx.x * kProlongChunk, n = (int64_t)NZp * NYp * NXp;
@@ -517,16 +537,16 @@ __global__ __launch_bounds__(kBlock) void k_prolongate_field(
     const float cy = cyp * LY / LYp;
     const float czp = (float)z * hZp;
     const float cz = czp * LZ / LZp;
-    axes[k][0] = sample_axis(ip, cx, hX, NX, bc);
-    axes[k][1] = sample_axis(ip, cy, hY, NY, bc);
-    axes[k][2] = sample_axis(ip, cz, hZ, NZ, bc);
+    axes[k][0] = sample_axis(IP, cx, hX, NX, bc);
+    axes[k][1] = sample_axis(IP, cy, hY, NY, bc);
+    axes[k][2] = sample_axis(IP, cz, hZ, NZ, bc);
   }
   __syncthreads();
   for (unsigned e = threadIdx.x; e < count; e += kBlock) {
     const unsigned k = (c0 + e) / (unsigned)C, c = c0 + e - k * (unsigned)C;
     const StridedFetch<I> f{u, (I)C, (I)c, NY, NX};
     float v[1];
-    sample_at<1>(ip, f, NZ, NY, NX, bc, axes[k][2], axes[k][1], axes[k][0], v);
+    sample_at<1>(IP, f, NZ, NY, NX, bc, axes[k][2], axes[k][1], axes[k][0], v);
     out[first + e] = v[0];
   }
 }
@@ -784,8 +804,8 @@ int svs_warp3d(const float* u, int C, const float* phi, int NZ, int NY, int NX, 
   SVS_REQUIRE_DIMS(NZ, NY, NX);
   SVS_REQUIRE(valid_bc(bdry) && valid_ip(interp), "Warping3D.forward: invalid interpolation/boundary type");
   const int64_t n = (int64_t)NZ * NY * NX;
-  const auto kernel = !narrow(n * C) ? k_warp<int64_t, 0> : C == 1 ? k_warp<unsigned, 1> : k_warp<unsigned, 0>;
-  kernel<<<grid_for(n, kBlock), kBlock, 0, (hipStream_t)stream>>>(u, C, phi, NZ, NY, NX, hZ, hY, hX, interp, bdry, out);
+  const auto kernel = SVS_PICK(k_warp, narrow(n * C), interp);
+  kernel<<<grid_for(n, kBlock), kBlock, 0, (hipStream_t)stream>>>(u, C, phi, NZ, NY, NX, hZ, hY, hX, bdry, out);
   SVS_LAUNCHED();
   return SVS_STATUS_OK;
 }
@@ -799,9 +819,9 @@ int svs_warp3d_cnn(const float* u, const float* phi, int B, int C, int NZ, int N
   const int64_t n = (int64_t)B * NZ * NY * NX;
   SVS_REQUIRE_WORKITEMS(n, "WarpingCNN3D.forward (batch x voxels)");
   const int64_t N = (int64_t)NZ * NY * NX;
-  const auto kernel = narrow(N) ? k_warp_cnn<unsigned> : k_warp_cnn<int64_t>;
+  const auto kernel = SVS_PICK(k_warp_cnn, narrow(N), interp);
   kernel<<<dim3(grid_for(N, kBlock), std::min(B, 65535)), kBlock, 0, (hipStream_t)stream>>>(
-      u, phi, B, C, NZ, NY, NX, hZ, hY, hX, interp, bdry, out);
+      u, phi, B, C, NZ, NY, NX, hZ, hY, hX, bdry, out);
   SVS_LAUNCHED();
   return SVS_STATUS_OK;
 }
@@ -816,7 +836,7 @@ int svs_propagate_masks(const float* mask_fwd, const float* mask_bwd, const floa
   SVS_REQUIRE_DIMS(NZ, NY, NX);
   SVS_REQUIRE(valid_bc(bdry) && valid_ip(interp), "mask propagation: invalid interpolation/boundary type");
   const int64_t N = (int64_t)NZ * NY * NX, M = N * C;
-  const auto kernel = narrow(N) ? k_propagate<unsigned> : k_propagate<int64_t>;
+  const auto kernel = SVS_PICK(k_propagate, narrow(N), interp);
   for (int t = 0; t < T; ++t) {
     const int to = t & 1, from = to ^ 1;
     ChainStep f{t ? scratch + (2 * from) * M : mask_fwd, flow_fwd + t * stride_fwd,
@@ -824,7 +844,7 @@ int svs_propagate_masks(const float* mask_fwd, const float* mask_bwd, const floa
     ChainStep b{t ? scratch + (2 * from + 1) * M : mask_bwd, flow_bwd + t * stride_bwd,
                 t + 1 < T ? scratch + (2 * to + 1) * M : nullptr, out_bwd + (int64_t)(T - 1 - t) * M,
                 t ? nullptr : out_bwd + (int64_t)T * M};
-    kernel<<<dim3(grid_for(N, kBlock), 2), kBlock, 0, (hipStream_t)stream>>>(f, b, C, NZ, NY, NX, hZ, hY, hX, interp, bdry,
+    kernel<<<dim3(grid_for(N, kBlock), 2), kBlock, 0, (hipStream_t)stream>>>(f, b, C, NZ, NY, NX, hZ, hY, hX, bdry,
                                                                            threshold);
     SVS_LAUNCHED();
   }
@@ -872,10 +892,9 @@ int svs_prolongate3d(const float* u, int C, int NZ, int NY, int NX, float LZ, fl
   // A thread per voxel for few channels: nothing is gained by sharing a
   // coordinate among lanes there, and the table would outgrow the LDS.
   const bool field = C >= kProlongChannels && chunks < ((int64_t)1 << 31);
-  const auto kernel = field ? (lean ? k_prolongate_field<unsigned> : k_prolongate_field<int64_t>)
-                            : (lean ? k_prolongate<unsigned> : k_prolongate<int64_t>);
+  const auto kernel = field ? SVS_PICK(k_prolongate_field, lean, interp) : SVS_PICK(k_prolongate, lean, interp);
   kernel<<<field ? (int)chunks : grid_for(n, kBlock), kBlock, 0, (hipStream_t)stream>>>(
-      u, C, NZ, NY, NX, LZ, LY, LX, hZ, hY, hX, NZp, NYp, NXp, LZp, LYp, LXp, hZp, hYp, hXp, interp, bdry, out);
+      u, C, NZ, NY, NX, LZ, LY, LX, hZ, hY, hX, NZp, NYp, NXp, LZp, LYp, LXp, hZp, hYp, hXp, bdry, out);
   SVS_LAUNCHED();
   return SVS_STATUS_OK;
 }
