@@ -966,6 +966,11 @@ __global__ __launch_bounds__(64) void k_stats_reduce(const float4* __restrict__ 
 }
 
 // ============================================================ host plan
+// Work-group extent (ring included) and planes per tile of the marching sweep.
+struct SweepShape {
+  int bx, by, cz;
+};
+
 struct LevelPlan {
   std::vector<LevelDesc> host;   // per instance
   LevelDesc* dev = nullptr;      // table in the workspace
@@ -1009,6 +1014,9 @@ struct LevelPlan {
   int* rest_dev = nullptr;
   SweepTile* rest_tiles = nullptr;
   int nrest_tiles = 0;
+  SweepShape rest_shape{};  // the marching tiles that suit them alone
+  int rest_threads = 0;
+  size_t rest_lds = 0;
 };
 
 }  // namespace svs
@@ -1088,9 +1096,6 @@ static size_t sweep_lds_bytes(int bx, int by) {
 // voxels wide and use at most bx * by threads; each instance gets its own tile
 // from it (inst_tile), so volumes of different widths in one launch all march
 // full (or evenly split) rows.  For NX == bx - 2 the tile is exactly bx x by.
-struct SweepShape {
-  int bx, by, cz;
-};
 
 static void inst_tile(const LevelDesc& d, int bx, int by, int& tbx, int& tby) {
   const int txmax = bx - 2;
@@ -1200,13 +1205,50 @@ static std::string tune_key(const svs_tvl1_params& P, const LevelPlan& L) {
   return k;
 }
 
+// The work of the busiest CU under a tile shape: the planes a work-group marches
+// (two more than it owns), times the threads of the CU's work-groups plus the 300
+// that a plane's latency is worth.  A count of work-groups just past a multiple
+// of the 256 CUs costs a whole round.  Of some 150 tiles timed for each of eleven
+// levels (one to nineteen volumes of 5 to 8 10^5 voxels) the one of least work was
+// the fastest or within 7 %.
+static double busiest_cu(const LevelPlan& L, const SweepShape& s) {
+  return (s.cz + 2.0) * ((count_tiles(L, s.bx, s.by, s.cz) + 255) / 256 * (s.bx * s.by) + 300);
+}
+static SweepShape one_round_shape(const LevelPlan& L, int maxNX) {
+  SweepShape best{0, 0, 0};
+  double least = 0.0;
+  int maxNZ = 0;
+  for (auto& d : L.host) maxNZ = std::max(maxNZ, d.NZ);
+  for (int n = (maxNX + 63) / 64; (maxNX + n - 1) / n >= 24; ++n) {
+    const int bx = (maxNX + n - 1) / n + 2;
+    for (int by = 8; by <= 16; ++by) {
+      if (bx * by > 832 || !shape_ok(L, bx, by, 1)) continue;
+      for (int cz : {2, 4, 6, 8, 12, 16, 24, 32}) {
+        if (cz > maxNZ && cz > 2) break;
+        const SweepShape s{bx, by, cz};
+        const double work = busiest_cu(L, s);
+        if (best.bx == 0 || work < least) {
+          least = work;
+          best = s;
+        }
+      }
+    }
+  }
+  return best;
+}
+
 // Default sweep shape policy of a level, by its voxel count (all instances).
 // Measured on MI355X with the autotuner: batches of large volumes run best
 // with full-row tiles of ~900 threads marching ~40 planes (68 x 80^3:
 // 82 x 11, 40 planes); mid-size levels with rows up to 64 wide and ~600
 // work-groups (68 x 40^3: 42 x 10, 20 planes); a single volume of 10^5..10^6
 // voxels with half rows marching 2 planes (80^3: 42 x 11); small levels are
-// latency-bound and want many small work-groups marching one plane.
+// latency-bound and want many small work-groups marching one plane.  What the
+// block-resident sweep does not hold, single volumes beyond 520,000 voxels and
+// batches of wide ones, takes the tile that one_round_shape finds: microseconds
+// per iteration with the rules here and with it, 64 x 96 x 96 31.0 and 26.2, 48 x
+// 128 x 128 40.4 and 32.4, 70 x 100 x 108 37.6 and 32.5, 25 x 128 x 180 31.5 and
+// 26.8, six 48 x 128 x 128 196 and 187.
 static void choose_sweep_shape(const svs_tvl1_params& P, LevelPlan& L, int ninst) {
   (void)ninst;
   int maxNX = 0;
@@ -1224,6 +1266,8 @@ static void choose_sweep_shape(const svs_tvl1_params& P, LevelPlan& L, int ninst
       return;
     }
   }
+  const bool rounds = bx <= 0 && by <= 0 && cz <= 0 && vox < ((int64_t)8 << 20) &&
+                      (vox > ((int64_t)1 << 20) ? maxNX > 64 : vox > ((int64_t)512 << 10));
   int maxtx, budget, minz, target;
   if (vox >= ((int64_t)8 << 20)) { maxtx = 128; budget = 910; minz = 40; target = 1024; }
   else if (vox >= ((int64_t)1 << 20)) { maxtx = 64; budget = 448; minz = 4; target = 600; }
@@ -1244,6 +1288,12 @@ static void choose_sweep_shape(const svs_tvl1_params& P, LevelPlan& L, int ninst
   }
   if (cz <= 0) cz = default_cz(L, bx, by, target, minz);
   L.bx = bx; L.by = by; L.cz = cz;
+  if (rounds) {  // where it promises a tenth
+    const SweepShape best = one_round_shape(L, maxNX);
+    if (best.bx && busiest_cu(L, best) < 0.9 * busiest_cu(L, SweepShape{bx, by, cz})) {
+      L.bx = best.bx; L.by = best.by; L.cz = best.cz;
+    }
+  }
 }
 
 // Tile extent of one instance for the block-resident sweep, or false when it
@@ -1550,8 +1600,12 @@ static int plan_layout(svs_plan* pl, char* base, size_t* total_out) {
         for (auto& b : L.blk_launches) tiles += b.tiles;
         L.blk_tiles_dev = (BlockTile*)take(sizeof(BlockTile) * tiles);
         if (!L.rest.empty()) {
+          LevelPlan R;
+          for (int k : L.rest) R.host.push_back(L.host[k]);
+          choose_sweep_shape(P, R, (int)L.rest.size());
+          L.rest_shape = SweepShape{R.bx, R.by, R.cz};
           L.rest_dev = (int*)take(sizeof(int) * L.rest.size());
-          L.rest_tiles = (SweepTile*)take(sizeof(SweepTile) * cap);
+          L.rest_tiles = (SweepTile*)take(sizeof(SweepTile) * count_tiles(R, R.bx, R.by, R.cz));
         }
         for (auto& b : L.blk_launches)  // whole rounds of the 8 XCDs' 4 shader engines
           pl->blk_need = std::max(pl->blk_need, (b.tiles + 31) / 32 * 32);
@@ -1775,22 +1829,22 @@ static int upload_tiles(svs_plan* pl, int s, hipStream_t st) {
     LevelPlan& L = pl->levels[s];
     L.ntiles = count_tiles(L, L.bx, L.by, L.cz);
     SVS_REQUIRE(L.ntiles <= L.tile_capacity, "tile table overflow (%d > %d)", L.ntiles, L.tile_capacity);
-    L.threads = 0;
-    L.lds = 0;
     // The tiles of the listed instances in launch order.
-    auto tiles_of = [&](const std::vector<int>& insts) {
+    auto tiles_of = [&](const std::vector<int>& insts, const SweepShape& shape, int& threads, size_t& lds) {
+      threads = 0;
+      lds = 0;
       std::vector<SweepTile> natural;
       for (int k : insts) {
         const LevelDesc& d = L.host[k];
         int tbx, tby;
-        inst_tile(d, L.bx, L.by, tbx, tby);
-        L.threads = std::max(L.threads, tbx * tby);
-        L.lds = std::max(L.lds, sweep_lds_bytes(tbx, tby));
+        inst_tile(d, shape.bx, shape.by, tbx, tby);
+        threads = std::max(threads, tbx * tby);
+        lds = std::max(lds, sweep_lds_bytes(tbx, tby));
         const int tx = tbx - 2, ty = tby - 2;
-        for (int z0 = 0; z0 < d.NZ; z0 += L.cz)
+        for (int z0 = 0; z0 < d.NZ; z0 += shape.cz)
           for (int y0 = 0; y0 < d.NY; y0 += ty)
             for (int x0 = 0; x0 < d.NX; x0 += tx) {
-              const int z1 = std::min(d.NZ, z0 + L.cz);
+              const int z1 = std::min(d.NZ, z0 + shape.cz);
               natural.push_back(SweepTile{k, x0 | (y0 << 16), z0 | (z1 << 16), tbx | (tby << 16)});
             }
       }
@@ -1810,10 +1864,10 @@ static int upload_tiles(svs_plan* pl, int s, hipStream_t st) {
     };
     std::vector<int> every(pl->ninst);
     for (int k = 0; k < pl->ninst; ++k) every[k] = k;
-    const std::vector<SweepTile> tiles = tiles_of(every);
+    const std::vector<SweepTile> tiles = tiles_of(every, SweepShape{L.bx, L.by, L.cz}, L.threads, L.lds);
     std::vector<SweepTile> rest;
     if (L.rest_tiles) {
-      rest = tiles_of(L.rest);
+      rest = tiles_of(L.rest, L.rest_shape, L.rest_threads, L.rest_lds);
       L.nrest_tiles = (int)rest.size();
       SVS_HIP(hipMemcpyAsync(L.rest_tiles, rest.data(), sizeof(SweepTile) * rest.size(), hipMemcpyHostToDevice, st));
     }
@@ -1844,12 +1898,13 @@ struct SweepScalars {
 template <int BC, bool ANISO, bool STATS, bool EXT>
 static void launch_sweep_s(const LevelPlan& L, int parity, const SweepScalars& a, float4* part, hipStream_t st) {
   const SweepTile* tiles = a.rest ? L.rest_tiles : L.tiles;
-  const int ntiles = a.rest ? L.nrest_tiles : L.ntiles;
+  const int ntiles = a.rest ? L.nrest_tiles : L.ntiles, threads = a.rest ? L.rest_threads : L.threads;
+  const size_t lds = a.rest ? L.rest_lds : L.lds;
   if (L.unit_h)
-    hipLaunchKernelGGL((k_sweep<BC, ANISO, true, STATS, EXT>), dim3(ntiles), dim3(L.threads), L.lds, st, L.dev,
+    hipLaunchKernelGGL((k_sweep<BC, ANISO, true, STATS, EXT>), dim3(ntiles), dim3(threads), lds, st, L.dev,
                        tiles, parity, a.sg, a.ta, a.fac, a.wtv, a.hub, a.eps, a.theta, a.zfirst, part);
   else
-    hipLaunchKernelGGL((k_sweep<BC, ANISO, false, STATS, EXT>), dim3(ntiles), dim3(L.threads), L.lds, st,
+    hipLaunchKernelGGL((k_sweep<BC, ANISO, false, STATS, EXT>), dim3(ntiles), dim3(threads), lds, st,
                        L.dev, tiles, parity, a.sg, a.ta, a.fac, a.wtv, a.hub, a.eps, a.theta, a.zfirst, part);
 }
 
