@@ -486,8 +486,9 @@ def main():
                      "traffic_per_level": traffic_detail["per_level"] if traffic_detail else None,
                      "traffic_over_algorithmic_per_level": (traffic_detail["per_level_over_algorithmic"]
                                                             if traffic_detail else None),
-                     "kernel": "k_sweep (fused primal-dual sweep; k_sweep_resident, all iterations of a warp in "
-                               "one launch, at levels of at most 2048 voxels per instance)",
+                     "kernel": "k_sweep (marching primal-dual sweep, one iteration per launch, timed by itself; k_sweep_resident "
+                               "at levels of at most 2048 voxels per instance). The step runs k_sweep_block, all "
+                               "iterations of a warp in one launch, wherever an instance fits the chip",
                      "bytes_per_launch_avg": int(avg_bytes), "us_per_launch_avg": round(avg_ms * 1e3, 2),
                      "level0_GBps": round(level0_gbps, 1),
                      "us_per_launch_by_level": [round(v * 1e3, 2) for v in sweep_ms]},

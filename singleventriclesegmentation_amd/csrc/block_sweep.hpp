@@ -63,7 +63,7 @@ constexpr int kBlkCapacity = 512;       // work-groups the device holds at once:
 
 // Per V voxels per thread: LDS words of one u component with its halo and of
 // one r component with the halo along its axis, and chunks of 64 exchange
-// entries per wave.  For V = 2, 76 KiB of LDS: two work-groups per CU.
+// entries per wave.  For V = 2, 75 KiB of LDS: two work-groups per CU.
 template <int V> struct BlkCap;
 template <> struct BlkCap<1> { static constexpr int U = 1152, R = 768, H = 3; };
 template <> struct BlkCap<2> { static constexpr int U = 2048, R = 1440, H = 4; };
