@@ -318,7 +318,8 @@ int svs_tvl1_plan_blocks(const svs_plan* plan, int level, int* out);
  * work-group alone, slowly and with the same results; the plan's later runs
  * then use the marching sweep, until mode -1 of svs_tvl1_plan_set_resident.
  * That happens only when something keeps the device from holding an
- * instance's work-groups at the same time, such as another process's kernels.
+ * instance's work-groups at the same time.  One process per device runs the
+ * block-resident sweep; plans of others march.
  * No reference counterpart. */
 int svs_tvl1_plan_set_wait_limit(svs_plan* plan, int microseconds, void* stream);
 

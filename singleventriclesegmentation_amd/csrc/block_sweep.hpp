@@ -47,8 +47,8 @@
 // (kCommit).  One that gives up before that decides the opposite (kRedo): all
 // of them leave, and the last redoes the instance's K iterations alone from
 // the untouched input state (slow, the same bits), and tells the host, which
-// goes back to the marching sweep (another process may hold part of the
-// device).
+// goes back to the marching sweep (work that it does not know of may hold part of
+// the device).
 //
 // Measured against the marching sweep, microseconds per iteration: one 80^3
 // 8.1 for 24.0 at K = 300 and 10.5 for 24.7 at K = 50 (the launch's fixed part

@@ -16,6 +16,13 @@
 //   p[2]       float[9][N]  SoA    dual, p[3c+d] = row c, derivative d
 //   z[2]       float[3][N]  SoA    over-relaxed point (extended model only)
 // J, SN and RG are shared by the levels of an instance (levels run in turn).
+#include <errno.h>
+#include <stddef.h>
+#include <stdio.h>
+#include <sys/socket.h>
+#include <sys/un.h>
+#include <unistd.h>
+
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -2021,8 +2028,39 @@ static int launch_blocks(const svs_plan* pl, const LevelPlan& L, int parity, hip
   return 0;
 }
 
+// Whether this process may run the block-resident sweep on a device: one process
+// at a time does, since the launches of two could each hold half of the device
+// and wait for the rest until the waits' limit.  The first to ask binds an
+// abstract socket named after the device's bus address, which the system frees
+// when the process ends; the others march (their work-groups wait for nobody, so they
+// do not hold up the first).  Where no socket can be had, the waits' limit decides.
+static bool claim_device(int device) {
+  static std::mutex mu;
+  static std::map<int, int> claims;  // device -> socket
+  std::lock_guard<std::mutex> lk(mu);
+  if (claims.count(device)) return true;
+  char bus[32] = "";
+  if (hipDeviceGetPCIBusId(bus, sizeof(bus), device) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  const int fd = socket(AF_UNIX, SOCK_DGRAM | SOCK_CLOEXEC, 0);
+  if (fd < 0) return true;
+  sockaddr_un name{};
+  name.sun_family = AF_UNIX;  // sun_path[0] = 0: the abstract namespace, no file
+  const int len = snprintf(name.sun_path + 1, sizeof(name.sun_path) - 1, "svsflow-blocks-%s", bus);
+  if (bind(fd, (const sockaddr*)&name, (socklen_t)(offsetof(sockaddr_un, sun_path) + 1 + len)) != 0) {
+    const bool taken = errno == EADDRINUSE;
+    close(fd);
+    return !taken;
+  }
+  claims[device] = fd;
+  return true;
+}
+
 // Switches the block-resident sweep off where the device does not hold
-// kBlkCapacity of its work-groups at once, and clears its counters.
+// kBlkCapacity of its work-groups at once or another process runs it, and
+// clears its counters.
 static int prepare_blocks(svs_plan* pl, hipStream_t st) {
   SVS_HIP(hipGetDevice(&pl->device));
   if (!pl->blk_need) return 0;
@@ -2036,7 +2074,7 @@ static int prepare_blocks(svs_plan* pl, hipStream_t st) {
     SVS_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)block_lds(L)));
     int per_cu = 0;
     SVS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlkThreads, block_lds(L)));
-    if (per_cu * cus < kBlkCapacity) {
+    if (per_cu * cus < kBlkCapacity || !claim_device(pl->device)) {
       L.blk_capable = L.blk_on = false;
       continue;
     }
@@ -2065,8 +2103,7 @@ static int prepare_blocks(svs_plan* pl, hipStream_t st) {
 // together.  Runs whose plan uses the block-resident sweep are kept in order of
 // enqueueing per device; a new one waits for every earlier run outside the
 // longest recent stretch that fits beside it, whatever streams and threads
-// they came from.  (Another process on the device is not seen here; then the
-// waits' time limit decides.)
+// they came from.
 static std::mutex g_runs_mu;
 static std::map<int, std::vector<svs_plan*>> g_runs;  // oldest first, each plan once
 

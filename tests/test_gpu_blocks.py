@@ -3,6 +3,9 @@ work-groups) gives the marching sweep's bits; the marching sweep equals the
 FP32 oracle's (test_gpu_solver.py, whose volumes of more than 2048 voxels also
 run block-resident)."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -111,3 +114,25 @@ def test_blocks_on_several_streams(dev):
         assert all(torch.equal(a, b) for a, b in zip(got, w))
         assert _blocks(plan)[0] == 1 and _blocks(plan)[4] == 0
         plan.close()
+
+
+_OTHER = """
+import ctypes, torch
+from singleventriclesegmentation_amd import _lib
+from singleventriclesegmentation_amd.solver import Plan, SolverConfig
+plan = Plan(SolverConfig(num_scales=1, max_warps=1, max_outer_iterations=3), [(20, 24, 22)])
+out = (ctypes.c_int * 5)()
+_lib.check(_lib.lib().svs_tvl1_plan_blocks(plan._h, 0, out))
+print("instances", out[0])
+"""
+
+
+def test_one_process_at_a_time_runs_blocks(dev):
+    """While this process's plans run block-resident, another one's march."""
+    plan, _ = _plan(dev, _config(3, 1, True), [(20, 24, 22)])
+    assert _blocks(plan)[0] == 1
+    repo = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    res = subprocess.run([sys.executable, "-c", _OTHER], cwd=repo, capture_output=True, text=True, timeout=100)
+    assert res.returncode == 0, res.stderr
+    assert "instances 0" in res.stdout
+    plan.close()
